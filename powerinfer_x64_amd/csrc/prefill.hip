@@ -1263,209 +1263,513 @@ __global__ __launch_bounds__(512, 1) void prefill_fa256_kernel(PrefillArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// prefill_f32_kernel: causal attention of a chunk of queries (f32 rows) over an
-// f32 KV pool, read through the sequence's page table (src/model/mod.rs:668
-// token loop over :1140-1190 with an f32 cache).  Products keep f32 accuracy
-// on the bf16 MFMA by splitting each f32 operand into bf16 hi + lo parts
-// (x = hi + lo to 16 significant bits, the exponent range of f32) and summing
-// hi.hi + hi.lo + lo.hi: three v_mfma_f32_16x16x32_bf16 per block.
+// prefill_f32_kernel / prefill_f32_256_kernel: causal attention of a chunk of
+// queries (f32 rows) over an f32 KV pool, read through the sequence's page table
+// (src/model/mod.rs:668 token loop over :1140-1190 with an f32 cache).  Products
+// keep f32 accuracy on the bf16 MFMA by splitting each f32 operand into bf16
+// hi + lo parts (x = hi + lo to 16 significant bits, the exponent range of f32)
+// and summing hi.hi + hi.lo + lo.hi: three MFMAs per block.
 //
-// A workgroup of 4 wavefronts covers 64 query rows of one query head; wave w
-// owns rows 16 w .. 16 w + 15.  Per 32-key tile (two pool pages):
-//   S^T[32 key x 16 q] = K . Q^T   (lane: query column c = lane % 16, keys 4 g + r)
-//   O^T[D x 16 q]     += V^T . P^T (P^T's contraction order matches the lane's keys)
-// K is staged in LDS as [key][dim] hi / lo rows, V as [dim][key] (the pool's V
-// block is already dim-major); the next tile's raw f32 pages are loaded into
-// registers while the current tile computes.
+// A workgroup of 8 wavefronts (two per SIMD) covers 128 query rows: HPW query
+// heads of one KV head x 128 / HPW rows, so that a key tile is read and split
+// once for all of them.  Per tile of TK keys (TK / 16 pool pages):
+//   S^T[keys x q] = K . Q^T   (a lane owns one query column)
+//   O^T[D x q]   += V^T . P^T (V^T's contraction order matches the lane's keys, so
+//                              P^T comes from the lane's own scores)
+// K sits in LDS as [key][dim] hi / lo rows, V as [dim][key] rows whose keys are
+// in the contraction's order.
+//
+// What bounds them on a long history: the matrix cores and the vector unit, 44 % and
+// about as much of a tile's cycles (128 rows x 64 keys at D 128: 1 536 MFMA cycles and
+// about 350 vector instructions a wavefront).  Two tile buffers and one barrier per
+// tile: the raw pages of tile t + 2 load into registers and tile t + 1 is split into
+// the free buffer while tile t computes; waves 0-3 split before they compute and waves
+// 4-7 after, so that the two wavefronts of a SIMD have vector and matrix work at the
+// same time.  Page ids are scalar loads, a tile ahead of the page loads that use them.
+// Against 64 rows a workgroup, 32-key tiles in one buffer and loads waited for where
+// they were issued: 1024 queries over 8192 keys, 32/32 heads, D 128 1574 -> 530 us (270
+// TFLOP/s, 810 of bf16 MFMA); a fresh 2048-token layer prompt 594 -> 190 us (32/8 heads
+// D 64 303 -> 102, 16/2 heads D 256 950 -> 204).
 // ---------------------------------------------------------------------------
-struct PrefillF32Args {
-    const float* q;         // [n_tok][hq][D], normalised and rotated
-    const float* kpool;     // f32 pool K blocks [D/4][16][4] of (page, kv head) i at kpool + i kstride
-    const float* vpool;     // f32 pool V blocks [D][16] at vpool + i vstride
-    size_t kstride, vstride;  // bytes
-    const int32_t* pt;      // the sequence's page-table row
-    float* out;             // [n_tok][hq][D]
-    const float* gate;      // optional [n_tok][hq][D]: out *= sigmoid(gate)
-    int n_tok, q_off, max_pages, n_pages, hq, hkv, group, gqa_mode;
-    float qk_scale;         // scale * log2(e)
-};
 
-template <int D>
-__global__ __launch_bounds__(256) void prefill_f32_kernel(PrefillF32Args a) {
-    constexpr int TK = 32;          // keys per tile (two pages)
-    // Row strides (bf16) chosen so that the 16-row x 4-chunk operand reads and the staging
-    // writes fall on distinct LDS banks: K rows of D + 16, V^T rows of 40 (80 bytes).
-    constexpr int KST = D + 16;     // K row stride (bf16)
-    constexpr int VST = TK + 8;     // V^T row stride (bf16)
-    constexpr int NF = 2 * TK * D / 4 / 256;  // float4 loads per thread per tile (K and V)
-    constexpr int NKS = D / 32;     // 32-dim steps of Q.K
-    constexpr int NDB = D / 16;     // 16-dim blocks of O^T
-    __shared__ __attribute__((aligned(16))) bf16 skh[TK * KST], skl[TK * KST];
-    __shared__ __attribute__((aligned(16))) bf16 svh[D * VST], svl[D * VST];
+// Position (in 16-byte chunks) of chunk c of row r in a tile of CH chunks a row.  The LDS
+// serves a 16-byte read 16 lanes at a time over 64 banks (16 chunks), and each such group
+// holds one row of every residue mod 16 (lanes 0-3, 12-15, 20-27 and their likes), so the
+// rows that start on one bank get XOR patterns of their own: 4.4 cycles a read measured,
+// 8.0 with half as many patterns.  M16: the 16-row operand's groups take two adjacent
+// chunks, rows 4-11 of their 16 the second one, which at 4 chunks a row needs the negated
+// pattern (4.4 against 8.0 cycles).
+template <int CH, bool M16>
+__device__ __forceinline__ int f32_chunk(int r, int c) {
+    const int x = CH >= 16 ? r & 15 : (r / (16 / CH)) & (CH - 1);
+    return r * CH + (c ^ (CH == 4 && M16 ? -x & 3 : x));
+}
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int g = lane >> 4, c = lane & 15;
-    const int qb = gridDim.x - 1 - blockIdx.x;  // heaviest (latest) query blocks first
-    const int head = blockIdx.y;
-    const int kvh = a.gqa_mode == 0 ? head % a.hkv : head / a.group;
-    const int L = a.q_off + a.n_tok;            // keys of the sequence after this chunk
-    const int p0 = qb * 64 + 16 * wave;         // this wave's first query row
-    const int wg_keys = min(L, a.q_off + qb * 64 + 64);
-    const int n_tiles = (wg_keys + TK - 1) / TK;
-    const int w_keys = min(L, a.q_off + p0 + 16);
-    const int w_tiles = p0 < a.n_tok ? (w_keys + TK - 1) / TK : 0;
-    const int qpos = p0 + c;
+// The key tiles of the two kernels: raw float4 pieces of the pool's pages, loaded into
+// registers a tile ahead (load), then split into hi / lo bf16 operands in LDS (stage).
+// Thread tid takes pieces tid + 512 j of the tile's pages (4 D pieces of K block
+// [D/4][16][4], then 4 D of V block [D][16]); in the V block the 64 pieces of a wavefront
+// are dealt dim-fastest, so that its LDS writes spread over the banks (8 cycles a write
+// against 16 in linear order).
+template <int D, int TK, bool M16>
+struct F32Tiles {
+    static constexpr int NPG = TK / 16;              // pages per tile
+    static constexpr int PF4 = 8 * D;                // pieces of a page
+    static constexpr int NF = TK * D / 2 / 512;      // pieces per thread and tile
+    static constexpr int KCH = D / 8, VCH = TK / 8;  // 16-byte chunks per K row / V^T row
+    typedef __attribute__((address_space(4))) const int32_t* const_i32p;
+    const_i32p pt;
+    const char* kpool;  // this KV head's blocks: page id's run starts at kpool + id * page_stride
+    size_t page_stride, voff;
+    int L, n_pages, tid;
+    int pid[NPG];
+    f32x4 pre[NF];
+    unsigned bad;  // pages of the loaded tile that are outside the pool: they hold no tokens (zeros)
 
-    // Q^T operand (B of K.Q^T): lane holds q[qpos][32 ks + 8 g .. +7] as hi / lo
-    bf16x8 qh[NKS], ql[NKS];
-    {
-        const bool ok = qpos < a.n_tok;
-        const float* qr = a.q + ((size_t)(ok ? qpos : 0) * a.hq + head) * D;
+    __device__ __forceinline__ void ids(int t, int (&id)[NPG]) const {
 #pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) {
-            f32x4 x0 = *reinterpret_cast<const f32x4*>(qr + 32 * ks + 8 * g);
-            f32x4 x1 = *reinterpret_cast<const f32x4*>(qr + 32 * ks + 8 * g + 4);
-            if (!ok) x0 = x1 = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float x = j < 4 ? x0[j] : x1[j - 4];
-                const bf16 h = to_bf16(x);
-                qh[ks][j] = h;
-                ql[ks][j] = to_bf16(x - (float)h);
-            }
+        for (int p = 0; p < NPG; ++p) {
+            const int lp = t * NPG + p;
+            id[p] = lp * 16 < L ? pt[lp] : -1;
         }
     }
-    f32x4 o[NDB];
-#pragma unroll
-    for (int i = 0; i < NDB; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float m_run = -1e30f, l_run = 0.f;
-
-    // Tile loads: float4 i of a tile (i = tid + 256 j) is K (i < 8 D) or V, of
-    // page i / (4 D) % 2; within a page block both are a linear copy.
-    f32x4 pre[NF];
-    auto load_tile = [&](int t) {
+    __device__ __forceinline__ void load() {
+        bad = 0;
 #pragma unroll
         for (int j = 0; j < NF; ++j) {
-            const int i = tid + 256 * j;
-            const bool isv = i >= 8 * D;
-            const int ii = isv ? i - 8 * D : i;
-            const int half = ii / (4 * D), ci = ii % (4 * D);
-            const int lp = 2 * t + half;
-            const int pid = lp < a.max_pages ? a.pt[lp] : -1;
-            const bool ok = lp * 16 < L && pid >= 0 && pid < a.n_pages;
-            const size_t bi = (size_t)(ok ? pid : 0) * a.hkv + kvh;
-            const float* base = reinterpret_cast<const float*>(
-                isv ? reinterpret_cast<const char*>(a.vpool) + bi * a.vstride
-                    : reinterpret_cast<const char*>(a.kpool) + bi * a.kstride);
-            pre[j] = ok ? *reinterpret_cast<const f32x4*>(base + 4 * ci) : f32x4{0.f, 0.f, 0.f, 0.f};
+            const int p = 512 * j / PF4, id = pid[p];
+            const bool ok = id >= 0 && id < n_pages;
+            if (!ok) bad |= 1u << p;
+            const char* page = kpool + (size_t)(ok ? id : 0) * page_stride;
+            const int w = tid + 512 * j % PF4, i = w - 4 * D;
+            pre[j] = *reinterpret_cast<const f32x4*>(
+                page + (i >= 0 ? voff + 16 * (size_t)((i & ~63) + 4 * (i & 15) + ((i >> 4) & 3)) : 16 * (size_t)w));
         }
-    };
-    auto stage_tile = [&]() {
+    }
+    __device__ __forceinline__ void stage(bf16x8* kh, bf16x8* kl, bf16x8* vh, bf16x8* vl) {
+        if (bad) {  // here and not at the load, whose result a select would wait for
+#pragma unroll
+            for (int j = 0; j < NF; ++j)
+                if (bad >> (512 * j / PF4) & 1) pre[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
 #pragma unroll
         for (int j = 0; j < NF; ++j) {
-            const int i = tid + 256 * j;
-            const bool isv = i >= 8 * D;
-            const int ii = isv ? i - 8 * D : i;
-            const int half = ii / (4 * D), ci = ii % (4 * D);
+            const int p = 512 * j / PF4, w = tid + 512 * j % PF4, i = w - 4 * D;
             bf16x4 h, l;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 h[e] = to_bf16(pre[j][e]);
                 l[e] = to_bf16(pre[j][e] - (float)h[e]);
             }
-            if (!isv) {  // K block [D/4][16][4]: dims 4 (ci / 16) .. +3 of token ci % 16
-                const int off = (16 * half + ci % 16) * KST + 4 * (ci / 16);
-                *reinterpret_cast<bf16x4*>(skh + off) = h;
-                *reinterpret_cast<bf16x4*>(skl + off) = l;
-            } else {     // V block [D][16]: tokens 4 (ci % 4) .. +3 of dim ci / 4
-                const int off = (ci / 4) * VST + 16 * half + 4 * (ci % 4);
-                *reinterpret_cast<bf16x4*>(svh + off) = h;
-                *reinterpret_cast<bf16x4*>(svl + off) = l;
+            if (i < 0) {  // dims 4 (w / 16) .. +3 of token w % 16
+                const int at = 2 * f32_chunk<KCH, M16>(16 * p + w % 16, w / 32) + (w / 16 & 1);
+                reinterpret_cast<bf16x4*>(kh)[at] = h;
+                reinterpret_cast<bf16x4*>(kl)[at] = l;
+            } else {
+                // tokens 4 m .. +3 of a dim.  Contraction order: 32-row operands take keys
+                // 16 p + 8 a + 4 b + r at slot 16 p + 8 b + 4 a + r; 16-row ones take key
+                // 32 n + 16 a + 4 b + r at slot 32 n + 8 b + 4 a + r.
+                const int dim = (i >> 6) * 16 + (i & 15), m = (i >> 4) & 3;
+                const int ch = M16 ? 4 * (p >> 1) + m : 2 * p + (m & 1), half = M16 ? p & 1 : m >> 1;
+                const int at = 2 * f32_chunk<VCH, M16>(dim, ch) + half;
+                reinterpret_cast<bf16x4*>(vh)[at] = h;
+                reinterpret_cast<bf16x4*>(vl)[at] = l;
             }
         }
+    }
+};
+
+// The barrier of the tile loops, without the compiler's wait for the loads in flight: LDS
+// writes are waited for here, global loads where their registers are used.
+__device__ __forceinline__ void f32_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+__device__ __forceinline__ void split_bf16(f32x4 x0, f32x4 x1, bf16x8& h, bf16x8& l) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float x = j < 4 ? x0[j] : x1[j - 4];
+        h[j] = to_bf16(x);
+        l[j] = to_bf16(x - (float)h[j]);
+    }
+}
+
+// Head dims 64 and 128, v_mfma_f32_32x32x16_bf16.  Wavefront w owns 32 query rows (row
+// group w % 4) and one 32-key half of each 64-key tile (w / 4): with 16 rows a wavefront and
+// whole tiles every wavefront would read the whole tile for half the rows, twice the LDS
+// bytes per MFMA.  The two halves' (max, sum, O) meet in LDS after the last tile.
+template <int D, int HPW>
+__global__ __launch_bounds__(512, 2) void prefill_f32_kernel(PrefillArgs a) {
+    constexpr int TK = 64;
+    constexpr int RG = 4 / HPW;               // row groups of 32 per head
+    constexpr int WROWS = 32 * RG;            // query rows per workgroup
+    constexpr int NKK = D / 16, NDT = D / 32;
+    typedef F32Tiles<D, TK, false> Tiles;
+    constexpr int KCH = Tiles::KCH, VCH = Tiles::VCH;
+    // per buffer: K hi, K lo (NK chunks each), V^T hi, V^T lo (as many: D VCH = TK KCH)
+    constexpr int NK = TK * KCH;
+    static_assert(NK == D * VCH, "tile");
+    __shared__ __attribute__((aligned(16))) bf16x8 lds[2][4 * NK];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 31, hh = lane >> 5;
+    const int rg = wave & 3, kh = wave >> 2;
+    const int per_kv = a.group / HPW;  // workgroups per KV head and query block
+    const int kvh = (int)blockIdx.x / per_kv;
+    const int head = head_of(kvh, ((int)blockIdx.x % per_kv) * HPW + rg / RG, a.hkv, a.group, a.gqa_mode);
+    // a head that does not exist (modulo map, n_q_heads not a multiple of n_kv_heads: HPW
+    // is 1) makes the whole workgroup leave, before any barrier
+    if (HPW == 1 && head >= a.hq) return;
+    const int qb = (int)gridDim.y - 1 - (int)blockIdx.y;  // heaviest (latest) query blocks first
+    const int S = a.S, L = a.Sk, q_off = a.q_off;         // L: keys of the sequence after this chunk
+    const int p0 = qb * WROWS + 32 * (rg % RG);           // this wave's first query row
+    const int qpos = p0 + r;
+    const int n_tiles = (min(L, q_off + qb * WROWS + WROWS) + TK - 1) / TK;
+    const int w_keys = p0 < S ? min(L, q_off + p0 + 32) : 0;  // keys this wave's rows attend
+
+    Tiles tl;
+    tl.pt = (typename Tiles::const_i32p)(uintptr_t)a.pt;
+    tl.kpool = a.kpool + (size_t)kvh * a.kstride;
+    tl.page_stride = (size_t)a.hkv * a.kstride;
+    tl.voff = a.vpool - a.kpool;
+    tl.L = L;
+    tl.n_pages = a.n_pages;
+    tl.tid = tid;
+    tl.ids(0, tl.pid);
+    tl.load();
+    tl.ids(1, tl.pid);
+
+    // Q^T operand: lane holds q[qpos][16 kk + 8 hh .. +7] as hi / lo
+    bf16x8 qh[NKK], ql[NKK];
+    {
+        const bool ok = qpos < S;
+        const float* qr = reinterpret_cast<const float*>(a.q) + ((size_t)(ok ? qpos : 0) * a.hq + head) * D;
+#pragma unroll
+        for (int kk = 0; kk < NKK; ++kk) {
+            f32x4 x0 = *reinterpret_cast<const f32x4*>(qr + 16 * kk + 8 * hh);
+            f32x4 x1 = *reinterpret_cast<const f32x4*>(qr + 16 * kk + 8 * hh + 4);
+            if (!ok) x0 = x1 = f32x4{0.f, 0.f, 0.f, 0.f};
+            split_bf16(x0, x1, qh[kk], ql[kk]);
+        }
+    }
+    f32x16 o[NDT];
+#pragma unroll
+    for (int i = 0; i < NDT; ++i) o[i] = f32x16{};
+    float m_run = -1e30f, l_run = 0.f;
+    auto mma = [](bf16x8 x, bf16x8 y, f32x16 acc) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, acc, 0, 0, 0);
     };
+    const float cs = a.qk_scale;
+    auto compute = [&](int k0, int buf) {  // keys k0 .. k0 + 31, rows 32 kh .. of the tile
+        f32x16 st = {};
+#pragma unroll
+        for (int kk = 0; kk < NKK; ++kk) {
+            const int at = f32_chunk<KCH, false>(32 * kh + r, 2 * kk + hh);
+            const bf16x8 xh = lds[buf][at], xl = lds[buf][NK + at];
+            st = mma(xh, qh[kk], st);
+            st = mma(xh, ql[kk], st);
+            st = mma(xl, qh[kk], st);
+        }
+        // operand reads two steps ahead of their MFMAs
+        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+        for (int kk = 0; kk < NKK - 2; ++kk) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
+        if (k0 + 32 > q_off + p0 || k0 + 32 > L) {  // reaches past a row's last key
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int key = k0 + 8 * (i >> 2) + 4 * hh + (i & 3);
+                if (key >= L || key > q_off + qpos) st[i] = -INFINITY;
+            }
+        }
+        float mx = st[0];
+#pragma unroll
+        for (int i = 1; i < 16; ++i) mx = fmaxf(mx, st[i]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        // the running max rises only when a score outgrows it by 2^8: P stays below that, and
+        // its hi + lo parts and the f32 sums keep their relative precision
+        if (__any(mx * cs > m_run + 8.0f)) {
+            const float m_new = fmaxf(m_run, mx * cs);
+            const float alpha = fast_exp2(m_run - m_new);
+            m_run = m_new;
+            l_run *= alpha;
+#pragma unroll
+            for (int i = 0; i < NDT; ++i) o[i] *= alpha;
+        }
+        // P^T operand of 16-key step s: slot 8 hh + j is the lane's score 8 s + j
+        bf16x8 ph[2], pl[2];
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float p = fast_exp2(__builtin_fmaf(st[8 * s + j], cs, -m_run));
+                l_run += p;
+                const bf16 h = to_bf16(p);
+                ph[s][j] = h;
+                pl[s][j] = to_bf16(p - (float)h);
+            }
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            bf16x8 xh[NDT], xl[NDT];
+#pragma unroll
+            for (int i = 0; i < NDT; ++i) {
+                const int at = f32_chunk<VCH, false>(32 * i + r, 4 * kh + 2 * s + hh);
+                xh[i] = lds[buf][2 * NK + at];
+                xl[i] = lds[buf][3 * NK + at];
+            }
+#pragma unroll
+            for (int i = 0; i < NDT; ++i) o[i] = mma(xh[i], ph[s], o[i]);
+#pragma unroll
+            for (int i = 0; i < NDT; ++i) o[i] = mma(xh[i], pl[s], o[i]);
+#pragma unroll
+            for (int i = 0; i < NDT; ++i) o[i] = mma(xl[i], ph[s], o[i]);
+        }
+    };
+
+    auto stage = [&](int buf) { tl.stage(lds[buf], lds[buf] + NK, lds[buf] + 2 * NK, lds[buf] + 3 * NK); };
+    stage(0);
+    if (1 < n_tiles) tl.load();
+    tl.ids(2, tl.pid);
+    f32_barrier();
+    for (int t = 0; t < n_tiles; ++t) {
+        const int buf = t & 1;
+        int nid[Tiles::NPG];
+        tl.ids(t + 3, nid);
+        auto next = [&]() {  // split tile t + 1, request tile t + 2
+            if (t + 1 < n_tiles) stage(buf ^ 1);
+            if (t + 2 < n_tiles) tl.load();
+#pragma unroll
+            for (int p = 0; p < Tiles::NPG; ++p) tl.pid[p] = nid[p];
+        };
+        const int k0 = t * TK + 32 * kh;
+        if (kh == 0) next();
+        if (k0 < w_keys) compute(k0, buf);
+        if (kh == 1) next();
+        f32_barrier();
+    }
+
+    // The two key halves of a row group: each wavefront hands the other the half of O that it
+    // does not write (dims 32 dt, dt / (NDT / 2) != kh) with its (max, sum).
+    l_run += __shfl_xor(l_run, 32, 64);
+    float* xch = reinterpret_cast<float*>(lds);  // [wave][NDT / 2][16][64], then [wave][2][64]
+    float* xml = xch + 8 * (NDT / 2) * 16 * 64;
+    static_assert((8 * (NDT / 2) * 16 * 64 + 8 * 2 * 64) * 4 <= (int)sizeof(lds), "exchange");
+#pragma unroll
+    for (int i = 0; i < NDT; ++i)
+        if ((i >= NDT / 2) != (kh == 1)) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) xch[((wave * (NDT / 2) + i % (NDT / 2)) * 16 + e) * 64 + lane] = o[i][e];
+        }
+    xml[(wave * 2) * 64 + lane] = m_run;
+    xml[(wave * 2 + 1) * 64 + lane] = l_run;
+    __syncthreads();
+    if (qpos >= S) return;
+    const int ow = wave ^ 4;
+    const float m_o = xml[(ow * 2) * 64 + lane], l_o = xml[(ow * 2 + 1) * 64 + lane];
+    const float M = fmaxf(m_run, m_o);
+    const float w_s = fast_exp2(m_run - M), w_o = fast_exp2(m_o - M);
+    const float inv = 1.0f / (w_s * l_run + w_o * l_o);
+    const float f_s = w_s * inv, f_o = w_o * inv;
+    const size_t row = (size_t)qpos * a.hq + head;
+    float* orow = a.out + row * D;
+#pragma unroll
+    for (int i = 0; i < NDT; ++i)
+        if ((i >= NDT / 2) == (kh == 1)) {
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const int d0 = 32 * i + 8 * b + 4 * hh;
+                f32x4 t;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    t[e] = o[i][4 * b + e] * f_s +
+                           xch[((ow * (NDT / 2) + i % (NDT / 2)) * 16 + 4 * b + e) * 64 + lane] * f_o;
+                if (a.gate) {
+                    const f32x4 gt = *reinterpret_cast<const f32x4*>(a.gate + row * D + d0);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) t[e] *= gate_sigmoid(gt[e]);
+                }
+                *reinterpret_cast<f32x4*>(orow + d0) = t;
+            }
+        }
+}
+
+// Head dim 256, v_mfma_f32_16x16x32_bf16: 32-row operands would take 256 registers for O and
+// Q^T alone.  Wavefront w owns 16 rows of head slot w / (8 / HPW) and attends whole tiles of
+// 32 keys (two buffers of a 64-key tile would need 256 KB).
+template <int HPW>
+__global__ __launch_bounds__(512, 2) void prefill_f32_256_kernel(PrefillArgs a) {
+    constexpr int D = 256, TK = 32;
+    constexpr int RW = 8 / HPW;               // row tiles of 16 per workgroup
+    constexpr int WROWS = 16 * RW;            // query rows per workgroup
+    constexpr int NKB = TK / 16;
+    constexpr int NKS = D / 32;               // 32-dim steps of Q.K
+    constexpr int NDB = D / 16;               // 16-dim blocks of O^T
+    typedef F32Tiles<D, TK, true> Tiles;
+    constexpr int KCH = Tiles::KCH, VCH = Tiles::VCH;
+    // per buffer: K hi, K lo (NK chunks each), V^T hi, V^T lo (as many: D VCH = TK KCH)
+    constexpr int NK = TK * KCH;
+    static_assert(NK == D * VCH, "tile");
+    __shared__ __attribute__((aligned(16))) bf16x8 lds[2][4 * NK];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, c = lane & 15;
+    const int per_kv = a.group / HPW;           // workgroups per KV head and query block
+    const int kvh = (int)blockIdx.x / per_kv;
+    const int head = head_of(kvh, ((int)blockIdx.x % per_kv) * HPW + wave / RW, a.hkv, a.group, a.gqa_mode);
+    if (HPW == 1 && head >= a.hq) return;  // as in prefill_f32_kernel
+    const int qb = (int)gridDim.y - 1 - (int)blockIdx.y;  // heaviest (latest) query blocks first
+    const int S = a.S, L = a.Sk, q_off = a.q_off;         // L: keys of the sequence after this chunk
+    const int p0 = qb * WROWS + 16 * (wave % RW);         // this wave's first query row
+    const int qpos = p0 + c;
+    const int n_tiles = (min(L, q_off + qb * WROWS + WROWS) + TK - 1) / TK;
+    const int w_keys = p0 < S ? min(L, q_off + p0 + 16) : 0;  // keys this wave's rows attend
+
+    Tiles tl;
+    tl.pt = (typename Tiles::const_i32p)(uintptr_t)a.pt;
+    tl.kpool = a.kpool + (size_t)kvh * a.kstride;
+    tl.page_stride = (size_t)a.hkv * a.kstride;
+    tl.voff = a.vpool - a.kpool;
+    tl.L = L;
+    tl.n_pages = a.n_pages;
+    tl.tid = tid;
+    tl.ids(0, tl.pid);
+    tl.load();
+    tl.ids(1, tl.pid);
+
+    // Q^T operand (B of K.Q^T): lane holds q[qpos][32 ks + 8 g .. +7] as hi / lo
+    bf16x8 qh[NKS], ql[NKS];
+    {
+        const bool ok = qpos < S;
+        const float* qr = reinterpret_cast<const float*>(a.q) + ((size_t)(ok ? qpos : 0) * a.hq + head) * D;
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) {
+            f32x4 x0 = *reinterpret_cast<const f32x4*>(qr + 32 * ks + 8 * g);
+            f32x4 x1 = *reinterpret_cast<const f32x4*>(qr + 32 * ks + 8 * g + 4);
+            if (!ok) x0 = x1 = f32x4{0.f, 0.f, 0.f, 0.f};
+            split_bf16(x0, x1, qh[ks], ql[ks]);
+        }
+    }
+    f32x4 o[NDB];
+#pragma unroll
+    for (int i = 0; i < NDB; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_run = -1e30f, l_run = 0.f;
     auto mma = [](bf16x8 x, bf16x8 y, f32x4 acc) {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, acc, 0, 0, 0);
     };
     const float cs = a.qk_scale;
-    load_tile(0);
-    for (int t = 0; t < n_tiles; ++t) {
-        __syncthreads();  // the previous tile's LDS reads are done
-        stage_tile();
-        if (t + 1 < n_tiles) load_tile(t + 1);
-        __syncthreads();
-        if (t >= w_tiles) continue;
-        // S^T for keys 16 kb + 4 g + r
-        f32x4 st[2];
+    auto compute = [&](int k0, int buf) {  // S^T for keys k0 + 16 kb + 4 g + r
+        f32x4 st[NKB];
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        for (int kb = 0; kb < NKB; ++kb) st[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int ks = 0; ks < NKS; ++ks) {
-                const int off = (16 * kb + c) * KST + 32 * ks + 8 * g;
-                const bf16x8 kh = *reinterpret_cast<const bf16x8*>(skh + off);
-                const bf16x8 kl = *reinterpret_cast<const bf16x8*>(skl + off);
-                acc = mma(kh, qh[ks], acc);
-                acc = mma(kh, ql[ks], acc);
-                acc = mma(kl, qh[ks], acc);
+        for (int ks = 0; ks < NKS; ++ks) {
+            bf16x8 xh[NKB], xl[NKB];
+#pragma unroll
+            for (int kb = 0; kb < NKB; ++kb) {
+                const int at = f32_chunk<KCH, true>(16 * kb + c, 4 * ks + g);
+                xh[kb] = lds[buf][at];
+                xl[kb] = lds[buf][NK + at];
             }
-            st[kb] = acc;
-        }
-        const int k0 = t * TK;
-        if (k0 + TK > a.q_off + p0 || k0 + TK > L) {  // the tile reaches past a row's last key
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
+            for (int kb = 0; kb < NKB; ++kb) st[kb] = mma(xh[kb], qh[ks], st[kb]);
+#pragma unroll
+            for (int kb = 0; kb < NKB; ++kb) st[kb] = mma(xh[kb], ql[ks], st[kb]);
+#pragma unroll
+            for (int kb = 0; kb < NKB; ++kb) st[kb] = mma(xl[kb], qh[ks], st[kb]);
+        }
+        if (k0 + TK > q_off + p0 || k0 + TK > L) {  // the tile reaches past a row's last key
+#pragma unroll
+            for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int key = k0 + 16 * kb + 4 * g + r;
-                    if (key >= L || key > a.q_off + qpos) st[kb][r] = -INFINITY;
+                    if (key >= L || key > q_off + qpos) st[kb][r] = -INFINITY;
                 }
         }
-        float mx = fmaxf(fmaxf(fmaxf(st[0][0], st[0][1]), fmaxf(st[0][2], st[0][3])),
-                         fmaxf(fmaxf(st[1][0], st[1][1]), fmaxf(st[1][2], st[1][3])));
+        float mx = st[0][0];
+#pragma unroll
+        for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) mx = fmaxf(mx, st[kb][r]);
         mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const float m_new = fmaxf(m_run, mx * cs);
-        const float alpha = fast_exp2(m_run - m_new);
-        m_run = m_new;
-        l_run *= alpha;
+        // the running max rises only when a score outgrows it by 2^8: P stays below that, and
+        // its hi + lo parts and the f32 sums keep their relative precision
+        if (__any(mx * cs > m_run + 8.0f)) {
+            const float m_new = fmaxf(m_run, mx * cs);
+            const float alpha = fast_exp2(m_run - m_new);
+            m_run = m_new;
+            l_run *= alpha;
 #pragma unroll
-        for (int i = 0; i < NDB; ++i) o[i] *= alpha;
-        // P^T operand: contraction slot 8 g + j is key 16 (j / 4) + 4 g + j % 4
+            for (int i = 0; i < NDB; ++i) o[i] *= alpha;
+        }
+        // P^T operand: slot 8 g + j is key 16 (j / 4) + 4 g + j % 4
         bf16x8 ph, pl;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const float p = fast_exp2(__builtin_fmaf(st[j >> 2][j & 3], cs, -m_new));
+            const float p = fast_exp2(__builtin_fmaf(st[j >> 2][j & 3], cs, -m_run));
             l_run += p;
             const bf16 h = to_bf16(p);
             ph[j] = h;
             pl[j] = to_bf16(p - (float)h);
         }
 #pragma unroll
-        for (int db = 0; db < NDB; ++db) {
-            const int off = (16 * db + c) * VST + 4 * g;
-            const bf16x4 h0 = *reinterpret_cast<const bf16x4*>(svh + off);
-            const bf16x4 h1 = *reinterpret_cast<const bf16x4*>(svh + off + 16);
-            const bf16x4 l0 = *reinterpret_cast<const bf16x4*>(svl + off);
-            const bf16x4 l1 = *reinterpret_cast<const bf16x4*>(svl + off + 16);
-            const bf16x8 vh = {h0[0], h0[1], h0[2], h0[3], h1[0], h1[1], h1[2], h1[3]};
-            const bf16x8 vl = {l0[0], l0[1], l0[2], l0[3], l1[0], l1[1], l1[2], l1[3]};
-            o[db] = mma(vh, ph, o[db]);
-            o[db] = mma(vh, pl, o[db]);
-            o[db] = mma(vl, ph, o[db]);
+        for (int d4 = 0; d4 < NDB; d4 += 4) {
+            bf16x8 xh[4], xl[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int at = f32_chunk<VCH, true>(16 * (d4 + i) + c, g);
+                xh[i] = lds[buf][2 * NK + at];
+                xl[i] = lds[buf][3 * NK + at];
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[d4 + i] = mma(xh[i], ph, o[d4 + i]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[d4 + i] = mma(xh[i], pl, o[d4 + i]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[d4 + i] = mma(xl[i], ph, o[d4 + i]);
         }
+    };
+
+    auto stage = [&](int buf) { tl.stage(lds[buf], lds[buf] + NK, lds[buf] + 2 * NK, lds[buf] + 3 * NK); };
+    stage(0);
+    if (1 < n_tiles) tl.load();
+    tl.ids(2, tl.pid);
+    f32_barrier();
+    for (int t = 0; t < n_tiles; ++t) {
+        const int buf = t & 1;
+        int nid[Tiles::NPG];
+        tl.ids(t + 3, nid);
+        auto next = [&]() {  // split tile t + 1, request tile t + 2
+            if (t + 1 < n_tiles) stage(buf ^ 1);
+            if (t + 2 < n_tiles) tl.load();
+#pragma unroll
+            for (int p = 0; p < Tiles::NPG; ++p) tl.pid[p] = nid[p];
+        };
+        if (wave < 4) next();
+        if (t * TK < w_keys) compute(t * TK, buf);
+        if (wave >= 4) next();
+        f32_barrier();
     }
+
     l_run += __shfl_xor(l_run, 16, 64);
     l_run += __shfl_xor(l_run, 32, 64);
-    if (qpos >= a.n_tok) return;
+    if (qpos >= S) return;
     const float inv = 1.0f / l_run;
-    const size_t ro = ((size_t)qpos * a.hq + head) * D;
-    float* orow = a.out + ro;
+    const size_t row = (size_t)qpos * a.hq + head;
+    float* orow = a.out + row * D;
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
         f32x4 t = o[db] * inv;
         if (a.gate) {
-            const f32x4 gt = *reinterpret_cast<const f32x4*>(a.gate + ro + 16 * db + 4 * g);
+            const f32x4 gt = *reinterpret_cast<const f32x4*>(a.gate + row * D + 16 * db + 4 * g);
 #pragma unroll
             for (int e = 0; e < 4; ++e) t[e] *= gate_sigmoid(gt[e]);
         }
@@ -1591,41 +1895,6 @@ void launch_d(const PrefillArgs& a, int hpw, int n_kv_heads, int seq_len, int ba
     }
 }
 }  // namespace
-
-hipError_t launch_prefill_f32(const KvGeom& g, const float* q, const int32_t* page_table,
-                              int32_t max_pages, int32_t q_off, int32_t n_tok, int32_t n_q_heads,
-                              int32_t gqa_mode, float scale, float* out, hipStream_t s,
-                              const float* gate) {
-    if (g.dtype != 0 || q_off < 0 || n_tok < 1 || max_pages < 1) return hipErrorInvalidValue;
-    const bool multiple = n_q_heads % g.n_kv_heads == 0;
-    if (!multiple && gqa_mode != 0) return hipErrorInvalidValue;
-    PrefillF32Args a;
-    a.q = q;
-    a.kpool = reinterpret_cast<const float*>(g.k);
-    a.vpool = reinterpret_cast<const float*>(g.v);
-    a.kstride = g.kstride;
-    a.vstride = g.vstride;
-    a.pt = page_table;
-    a.out = out;
-    a.gate = gate;
-    a.n_tok = n_tok;
-    a.q_off = q_off;
-    a.max_pages = max_pages;
-    a.n_pages = g.n_pages;
-    a.hq = n_q_heads;
-    a.hkv = g.n_kv_heads;
-    a.group = (n_q_heads + g.n_kv_heads - 1) / g.n_kv_heads;
-    a.gqa_mode = gqa_mode;
-    a.qk_scale = scale * kLog2e;
-    const dim3 grid((unsigned)((n_tok + 63) / 64), (unsigned)n_q_heads);
-    switch (g.head_dim) {
-        case 64: hipLaunchKernelGGL(prefill_f32_kernel<64>, grid, dim3(256), 0, s, a); break;
-        case 128: hipLaunchKernelGGL(prefill_f32_kernel<128>, grid, dim3(256), 0, s, a); break;
-        case 256: hipLaunchKernelGGL(prefill_f32_kernel<256>, grid, dim3(256), 0, s, a); break;
-        default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
 
 namespace {
 int cu_count() {
@@ -1865,6 +2134,59 @@ hipError_t launch_prefill_pool(const KvGeom& g, const void* q, int32_t q_f32, co
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || a.ksplit == 1) return e;
     return launch_merge(D, a, 1, q0, wrows, out, s);
+}
+
+hipError_t launch_prefill_f32(const KvGeom& g, const float* q, const int32_t* page_table,
+                              int32_t max_pages, int32_t q_off, int32_t n_tok, int32_t n_q_heads,
+                              int32_t gqa_mode, float scale, float* out, hipStream_t s,
+                              const float* gate) {
+    const int D = g.head_dim;
+    if (g.dtype != 0 || (D != 64 && D != 128 && D != 256) || q_off < 0 || n_tok < 1 || max_pages < 1)
+        return hipErrorInvalidValue;
+    // the kernel reads the row's ids of every key's page and takes one stride for both blocks
+    if ((long long)q_off + n_tok > (long long)max_pages * kPageTokens || g.kstride != g.vstride)
+        return hipErrorInvalidValue;
+    const bool multiple = n_q_heads % g.n_kv_heads == 0;
+    if (!multiple && gqa_mode != 0) return hipErrorInvalidValue;
+    PrefillArgs a{};
+    a.q = q;
+    a.out = out;
+    a.gate = gate;
+    a.S = n_tok;
+    a.Sk = q_off + n_tok;
+    a.q_off = q_off;
+    a.hq = n_q_heads;
+    a.hkv = g.n_kv_heads;
+    a.group = (n_q_heads + g.n_kv_heads - 1) / g.n_kv_heads;
+    a.causal = 1;
+    a.gqa_mode = gqa_mode;
+    a.qk_scale = scale * kLog2e;
+    a.pt = page_table;
+    a.kpool = static_cast<const char*>(g.k);
+    a.vpool = static_cast<const char*>(g.v);
+    a.kstride = g.kstride;
+    a.vstride = g.vstride;
+    a.n_pages = g.n_pages;
+    a.ksplit = 1;
+    const int hpw = !multiple ? 1 : a.group % 4 == 0 ? 4 : (a.group % 2 == 0 ? 2 : 1);
+    const int wrows = 128 / hpw;
+    const dim3 grid((unsigned)(g.n_kv_heads * (a.group / hpw)), (unsigned)((n_tok + wrows - 1) / wrows));
+#define PI_F32(DD)                                                                                \
+    switch (hpw) {                                                                                \
+        case 4: hipLaunchKernelGGL((prefill_f32_kernel<DD, 4>), grid, dim3(512), 0, s, a); break; \
+        case 2: hipLaunchKernelGGL((prefill_f32_kernel<DD, 2>), grid, dim3(512), 0, s, a); break; \
+        default: hipLaunchKernelGGL((prefill_f32_kernel<DD, 1>), grid, dim3(512), 0, s, a);       \
+    }
+    if (D == 256) {
+        switch (hpw) {
+            case 4: hipLaunchKernelGGL(prefill_f32_256_kernel<4>, grid, dim3(512), 0, s, a); break;
+            case 2: hipLaunchKernelGGL(prefill_f32_256_kernel<2>, grid, dim3(512), 0, s, a); break;
+            default: hipLaunchKernelGGL(prefill_f32_256_kernel<1>, grid, dim3(512), 0, s, a);
+        }
+    } else if (D == 128) PI_F32(128)
+    else PI_F32(64)
+#undef PI_F32
+    return hipGetLastError();
 }
 
 }  // namespace pi

@@ -1,0 +1,71 @@
+"""The f32 pool's prefill kernels (32-row workgroup tiles with two key halves at head dims 64
+and 128, 16-row ones at 256) at the edges of their tiles, against the oracle.
+
+Tolerance: an operand x is kept as bf16 hi + lo (relative error 2^-17), the lo.lo product is
+dropped (2^-16 of |q_i k_i|), so a score moves by at most e = 2^-15 scale sum_i |q_i k_i|, a
+softmax weight by a factor within exp(+-2 e), and the weights' and values' own splits add
+2^-15: |out - ref| <= (exp(2 e) - 1 + 2^-15) max |v| + f32 rounding (2^-20 max |v|).
+"""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as orc
+from tests.gpu_util import device, to_dev
+from tests.test_gpu_prefill_paged import Chunk
+
+pytestmark = pytest.mark.gpu
+
+
+def _bound(q, k, v):
+    hq, hkv, d = q.shape[1], k.shape[1], q.shape[2]
+    kk = np.abs(k[:, np.arange(hq) % hkv].astype(np.float64))  # modulo head map
+    e = 2.0 ** -15 * np.einsum("nhd,lhd->nlh", np.abs(q.astype(np.float64)), kk).max() / np.sqrt(d)
+    return (np.expm1(2 * e) + 2.0 ** -15 + 2.0 ** -20) * np.abs(v).max()
+
+
+def _check(c, out, rows, k=None, v=None):
+    q, kr, vr = c.prepared(f32=True)
+    k, v = (kr if k is None else k), (vr if v is None else v)
+    for i in rows:
+        ref = orc.attn_decode(q[i], k[:c.prev + i + 1], v[:c.prev + i + 1])
+        err, tol = float(np.abs(out[i] - ref).max()), _bound(q[i:i + 1], k[:c.prev + i + 1], v)
+        assert err <= tol, f"row {i}: max-abs {err} > {tol}"
+
+
+# rows around the 32-row groups and the 32 / 64 / 128-row blocks of 4, 2 and 1 heads a workgroup;
+# histories at and beside tiles, so that a key half holds no key of some rows
+@pytest.mark.parametrize("hq,hkv", [(8, 2), (4, 2), (3, 3), (5, 2)])
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("prev,n", [(0, 31), (0, 33), (31, 1), (63, 66), (64, 127), (97, 129)])
+def test_f32_prefill_tile_edges(prev, n, hq, hkv, d):
+    c = Chunk(np.random.default_rng(prev * 131 + n + hq + d), prev, n, hq, hkv, d)
+    out = c.gpu(device(), pool_dtype=torch.float32)
+    _check(c, out, sorted({0, n // 2, n - 1} | {r for r in (31, 32, 63, 64, 127, 128) if r < n}))
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_f32_prefill_max_rises_late(d):
+    """Scores that outgrow the running max tile after tile (the kernels raise it lazily)."""
+    c = Chunk(np.random.default_rng(d), 0, 200, 4, 2, d)
+    c.k *= np.linspace(0.2, 4.0, 200, dtype=np.float32)[:, None, None]
+    out = c.gpu(device(), pool_dtype=torch.float32)
+    _check(c, out, [0, 31, 63, 64, 130, 199])
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_f32_prefill_page_outside_the_pool(d):
+    """A page id outside the pool reads as zero keys and values."""
+    from powerinfer_x64_amd import runtime as rt
+    dev = device()
+    c = Chunk(np.random.default_rng(d + 1), 150, 40, 4, 2, d)
+    c.gpu(dev, pool_dtype=torch.float32)
+    q, k, v = c.prepared(f32=True)
+    row = c.row.copy()
+    row[3], row[9] = c.n_pages, -1
+    k, v = k.copy(), v.copy()
+    for p in (3, 9):
+        k[16 * p:16 * p + 16] = 0
+        v[16 * p:16 * p + 16] = 0
+    out = rt.attn_prefill_paged(dev, to_dev(q), c.pool, to_dev(row), c.prev).cpu().numpy()
+    _check(c, out, [0, 20, 39], k, v)
