@@ -214,3 +214,32 @@ def test_pool_rejects_bad_shapes():
     with pytest.raises(rt.InvalidArg):  # 4 q heads over 3 kv heads: the grouped map needs a multiple
         rt.attn_decode(dev, q, pool, torch.zeros((1, 1), dtype=torch.int32, device="cuda"),
                        torch.ones(1, dtype=torch.int32, device="cuda"), gqa_mode=1)
+
+
+@pytest.mark.parametrize("n_tok", [16, 130, 300, 513, 1025])
+@pytest.mark.parametrize("hq,hkv,d", [(5, 2, 64), (32, 8, 128), (9, 3, 256)])
+def test_prologue_head_groups_do_not_change_rows(n_tok, hq, hkv, d):
+    """One launch's token count picks how many workgroups share a token's heads; the rows and
+    pages are those of 15-token launches (every head group its own workgroup), which append K /
+    V per token and not by page: there a multiply and add may fuse otherwise, a rounding of
+    2^-24 in each of three products and sums of values up to twice the row's largest."""
+    from powerinfer_x64_amd import runtime as rt
+    dev = device()
+    rng = np.random.default_rng(n_tok + hq)
+    w = to_dev(rng.uniform(0.5, 1.5, d).astype(np.float32))
+    pages = (n_tok + 15) // 16
+    pt = to_dev(rng.permutation(pages).astype(np.int32)[None])
+    rows = [rng.standard_normal((1, n_tok, h, d)).astype(np.float32) for h in (hq, hkv, hkv)]
+    got = []
+    for step in (n_tok, 15):
+        pool = rt.KvPool(dev, pages, hkv, d, dtype=torch.float32)
+        q, k, v = (to_dev(r) for r in rows)
+        outs = []
+        for t in range(0, n_tok, step):
+            qs, ks, vs = (x[:, t:t + step].contiguous() for x in (q, k, v))
+            rt.attn_prologue(dev, qs, ks, vs, pool, pt, torch.tensor([t], dtype=torch.int32, device="cuda"), w, w,
+                             1e-6, d, 1e6, None)
+            outs.append((qs, ks))
+        got.append([torch.cat([o[i] for o in outs], 1) for i in (0, 1)] + list(pool.read(pt, 0, 0, n_tok)))
+    for a, b in zip(*got):
+        assert float((a - b).abs().max()) <= 3 * 2 * 2.0 ** -24 * float(b.abs().max())
