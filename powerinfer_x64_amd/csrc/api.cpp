@@ -779,6 +779,22 @@ int pi_gdn_decode(pi_handle h, const float* d_q, const float* d_k, const float* 
     return PI_OK;
 }
 
+// The chunked prefill on the handle's workspace, k_hd = v_hd = 128 (conv_*: a layer's conv
+// state to roll, see launch_gdn_prefill).
+static int gdn_prefill_ws(pi_handle h, const char* fn, const float* d_q, const float* d_k, const float* d_v,
+                          const float* d_beta, const float* d_g, float* d_state, float* d_out,
+                          int32_t n_tok, int32_t n_k_heads, int32_t n_v_heads, hipStream_t s,
+                          const float* conv_x, float* conv_state, int32_t conv_dim) {
+    int rc;
+    if ((rc = ws_begin(h, s, fn))) return rc;
+    const size_t need = pi::gdn_prefill_ws_floats(n_tok, n_k_heads, n_v_heads, 64);
+    if (need && (rc = grow(h, &h->gws.buf, &h->gws.capacity, need, s, "pi_gdn_prefill workspace", false))) return rc;
+    PI_HIP(h, pi::launch_gdn_prefill(d_q, d_k, d_v, d_beta, d_g, d_state, d_out, n_tok, n_k_heads, n_v_heads, 64,
+                                     h->gws, s, conv_x, conv_state, conv_dim),
+           fn);
+    return ws_end(h, s, fn);
+}
+
 int pi_gdn_prefill(pi_handle h, const float* d_q, const float* d_k, const float* d_v,
                    const float* d_beta, const float* d_g, float* d_state, float* d_out,
                    int32_t n_tok, int32_t n_k_heads, int32_t n_v_heads, int32_t k_hd, int32_t v_hd,
@@ -800,16 +816,8 @@ int pi_gdn_prefill(pi_handle h, const float* d_q, const float* d_k, const float*
                "pi_gdn_prefill");
         return PI_OK;
     }
-    if ((rc = ws_begin(h, s, "pi_gdn_prefill"))) return rc;
-    const size_t need = pi::gdn_prefill_ws_floats(n_tok, n_k_heads, n_v_heads, chunk);
-    if (need) {
-        rc = grow(h, &h->gws.buf, &h->gws.capacity, need, s, "pi_gdn_prefill workspace", false);
-        if (rc) return rc;
-    }
-    hipError_t e = pi::launch_gdn_prefill(d_q, d_k, d_v, d_beta, d_g, d_state, d_out, n_tok,
-                                          n_k_heads, n_v_heads, chunk, h->gws, s);
-    if (e != hipSuccess) return hip_fail(h, e, "pi_gdn_prefill");
-    return ws_end(h, s, "pi_gdn_prefill");
+    return gdn_prefill_ws(h, "pi_gdn_prefill", d_q, d_k, d_v, d_beta, d_g, d_state, d_out, n_tok, n_k_heads,
+                          n_v_heads, s, nullptr, nullptr, 0);
 }
 
 // ---- host-slice drop-ins -------------------------------------------------------------
@@ -1547,6 +1555,21 @@ static int gdn_layer_step(pi_handle h, pi_gdn_layer L, const float* dx, const fl
     if (rc) return rc;
     float *act = L->d_buf, *dq = act + n * C, *dk = dq + n * kd, *dv = dk + n * kd;
     float *db = dv + n * vd, *dg = db + n * nh;
+    if (n > 1 && pi::gdn_layer_in_ok(dx, L->d_conv_state, L->hk, L->hv, L->dk, L->dv, L->d_conv)) {
+        // conv, split and gates in one launch, then the recurrence, which rolls the conv state
+        PI_HIP(h, pi::launch_gdn_layer_in(dx, L->d_conv_state, L->d_w, dbr, dar, L->d_ssm_a, L->d_dt, dq, dk, dv,
+                                          db, dg, n_tokens, L->hk, L->hv, L->dk, L->dv, s),
+               "gdn layer");
+        if (L->dk == 128 && L->dv == 128) {
+            rc = gdn_prefill_ws(h, "gdn layer", dq, dk, dv, db, dg, L->d_state, dout, n_tokens, L->hk, L->hv, s,
+                                dx, L->d_conv_state, (int32_t)C);
+        } else {
+            PI_HIP(h, pi::launch_gdn_conv_state(dx, L->d_conv_state, n_tokens, (int32_t)C, L->d_conv, s), "gdn layer");
+            rc = pi_gdn_prefill(h, dq, dk, dv, db, dg, L->d_state, dout, n_tokens, L->hk, L->hv, L->dk, L->dv, 64, sv);
+        }
+        if (rc) return rc;
+        return pi_gdn_rmsnorm_gated(h, dout, dz, L->d_norm, n_tokens, L->hv, L->dv, L->eps, sv);
+    }
     if ((rc = pi_gdn_conv1d(h, dx, L->d_conv_state, L->d_w, act, 1, n_tokens, (int32_t)C, L->d_conv, sv)))
         return rc;
     if (n == 1) {  // one token's row already holds q, k and v back to back

@@ -18,6 +18,14 @@ namespace {
 constexpr int DK = 128;
 constexpr int DV = 128;
 
+__device__ __forceinline__ void gate_one(float beta_raw, float a_raw, float ssm_a, float dt_bias,
+                                         float* beta, float* g) {
+    *beta = 1.0f / (1.0f + expf(-beta_raw));
+    const float sp_in = a_raw + dt_bias;
+    const float sp = sp_in > 10.0f ? sp_in : logf(1.0f + expf(sp_in));
+    *g = ssm_a * sp;
+}
+
 __global__ __launch_bounds__(256) void gdn_gates_kernel(const float* __restrict__ beta_raw,
                                                         const float* __restrict__ a_raw,
                                                         const float* __restrict__ ssm_a,
@@ -28,10 +36,7 @@ __global__ __launch_bounds__(256) void gdn_gates_kernel(const float* __restrict_
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= n_tok * hv) return;
     const int h = idx % hv;
-    beta[idx] = 1.0f / (1.0f + expf(-beta_raw[idx]));
-    const float sp_in = a_raw[idx] + dt_bias[h];
-    const float sp = sp_in > 10.0f ? sp_in : logf(1.0f + expf(sp_in));
-    g[idx] = ssm_a[h] * sp;
+    gate_one(beta_raw[idx], a_raw[idx], ssm_a[h], dt_bias[h], &beta[idx], &g[idx]);
 }
 
 // Depthwise causal conv1d + SiLU over the QKV channels (src/model/mod.rs:750-776).
@@ -64,26 +69,16 @@ __global__ __launch_bounds__(256) void gdn_conv1d_kernel(const float* __restrict
 }
 
 // The model's case, d_conv = 4 with 4 | conv_dim and 16-byte aligned rows: a
-// thread owns channels 4 c4 .. 4 c4 + 3 of one sequence and walks kConvTok
-// tokens with the three previous rows of X_ext in registers, so every input
-// is read once (16 bytes) and its taps once per thread; the 3-D grid needs no
-// index division.  Same arithmetic per element as gdn_conv1d_kernel.
-constexpr int kConvTok = 32;
-__global__ __launch_bounds__(256) void gdn_conv1d_k4_kernel(const float* __restrict__ x,
-                                                            const float* __restrict__ state,
-                                                            const float* __restrict__ w,
-                                                            float* __restrict__ out, int n_tok,
-                                                            int conv_dim) {
-    const int c4 = blockIdx.x * 256 + threadIdx.x;
-    if (4 * c4 >= conv_dim) return;
-    const int t0 = blockIdx.y * kConvTok, sq = blockIdx.z;
-    const size_t q4 = (size_t)conv_dim / 4;  // 16-byte groups per row
-    const f32x4* xs = reinterpret_cast<const f32x4*>(x + (size_t)sq * n_tok * conv_dim) + c4;
-    const f32x4* ss = reinterpret_cast<const f32x4*>(state + (size_t)sq * 3 * conv_dim) + c4;
-    f32x4* os = reinterpret_cast<f32x4*>(out + (size_t)sq * n_tok * conv_dim) + c4;
+// thread owns channels 4 c4 .. 4 c4 + 3 of one sequence and walks tokens t0 .. t1 - 1 with
+// the three previous rows of X_ext in registers, so every input is read once (16 bytes)
+// and its taps once per thread.  Bound by memory: the rows of four tokens are requested
+// before any is used.  Same arithmetic per element as gdn_conv1d_kernel.  xs / ss / wr: the
+// thread's column of x, of the state and its taps; os: its output column, oq groups a row.
+__device__ __forceinline__ void conv4_walk(const f32x4* __restrict__ xs, const f32x4* __restrict__ ss,
+                                           const f32x4* __restrict__ wr, f32x4* __restrict__ os,
+                                           size_t q4, size_t oq, int t0, int t1) {
     f32x4 wk[4];  // wk[k][e] = tap k of channel 4 c4 + e
     {
-        const f32x4* wr = reinterpret_cast<const f32x4*>(w) + 4 * c4;
         f32x4 wc[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) wc[e] = wr[e];
@@ -92,22 +87,80 @@ __global__ __launch_bounds__(256) void gdn_conv1d_k4_kernel(const float* __restr
     }
     auto ext = [&](int r) { return r < 3 ? ss[(size_t)r * q4] : xs[(size_t)(r - 3) * q4]; };
     f32x4 a = ext(t0), b = ext(t0 + 1), c = ext(t0 + 2);
-    const int t1 = min(n_tok, t0 + kConvTok);
-    for (int t = t0; t < t1; ++t) {
-        const f32x4 d = xs[(size_t)t * q4];  // X_ext row t + 3
-        f32x4 val = {0.f, 0.f, 0.f, 0.f};
-        val += wk[0] * a;
-        val += wk[1] * b;
-        val += wk[2] * c;
-        val += wk[3] * d;
-        f32x4 o;
+    for (int t = t0; t < t1; t += 4) {
+        f32x4 d[4];  // X_ext rows t + 3 ..
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = val[e] / (1.0f + expf(-val[e]));
-        os[(size_t)t * q4] = o;
-        a = b;
-        b = c;
-        c = d;
+        for (int i = 0; i < 4; ++i) d[i] = xs[(size_t)min(t + i, t1 - 1) * q4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            f32x4 val = {0.f, 0.f, 0.f, 0.f};
+            val += wk[0] * a;
+            val += wk[1] * b;
+            val += wk[2] * c;
+            val += wk[3] * d[i];
+            f32x4 o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = val[e] / (1.0f + expf(-val[e]));
+            if (t + i < t1) os[(size_t)(t + i) * oq] = o;
+            a = b;
+            b = c;
+            c = d[i];
+        }
     }
+}
+
+__global__ __launch_bounds__(256) void gdn_conv1d_k4_kernel(const float* __restrict__ x,
+                                                            const float* __restrict__ state,
+                                                            const float* __restrict__ w,
+                                                            float* __restrict__ out, int n_tok,
+                                                            int conv_dim, int toks) {
+    const int c4 = blockIdx.x * 256 + threadIdx.x;
+    if (4 * c4 >= conv_dim) return;
+    const int t0 = blockIdx.y * toks, sq = blockIdx.z;
+    const size_t q4 = (size_t)conv_dim / 4;  // 16-byte groups per row
+    conv4_walk(reinterpret_cast<const f32x4*>(x + (size_t)sq * n_tok * conv_dim) + c4,
+               reinterpret_cast<const f32x4*>(state + (size_t)sq * 3 * conv_dim) + c4,
+               reinterpret_cast<const f32x4*>(w) + 4 * c4,
+               reinterpret_cast<f32x4*>(out + (size_t)sq * n_tok * conv_dim) + c4, q4, q4, t0,
+               min(n_tok, t0 + toks));
+}
+
+// A layer prompt's conv1d + SiLU and gates in one launch: the conv's q, k and v columns go to
+// the rows that the recurrence reads (q, k [n_tok][kd], v [n_tok][vd]: the activation in one
+// [n_tok][conv_dim] array took three copies, 41 us of a 4096-token prompt at 16/32 heads),
+// and the workgroups past the conv's (blockIdx.y >= ny) compute beta and g
+// (gdn_gates_kernel's arithmetic).  Bound by memory: 51 us for that prompt's 269 MB; the
+// layer step went from 313 to 245 us in four launches instead of nine.
+struct GdnLayerIn {
+    const float *x, *state, *w, *beta_raw, *a_raw, *ssm_a, *dt_bias;
+    float *q, *k, *v, *beta, *g;
+    int n_tok, conv_dim, kd, vd, hv;
+};
+__global__ __launch_bounds__(256) void gdn_layer_in_kernel(GdnLayerIn p, int toks, int ny) {
+    if ((int)blockIdx.y >= ny) {
+        const long long n = (long long)p.n_tok * p.hv;
+        for (long long i = ((long long)(blockIdx.y - ny) * gridDim.x + blockIdx.x) * 256 + threadIdx.x; i < n;
+             i += (long long)(gridDim.y - ny) * gridDim.x * 256)
+            gate_one(p.beta_raw[i], p.a_raw[i], p.ssm_a[i % p.hv], p.dt_bias[i % p.hv], &p.beta[i], &p.g[i]);
+        return;
+    }
+    const int c4 = blockIdx.x * 256 + threadIdx.x, col = 4 * c4;
+    if (col >= p.conv_dim) return;
+    const int t0 = blockIdx.y * toks;
+    const int row = col < 2 * p.kd ? p.kd : p.vd;  // 4 | kd: a group of four columns is one operand's
+    float* o = col < p.kd ? p.q + col : col < 2 * p.kd ? p.k + (col - p.kd) : p.v + (col - 2 * p.kd);
+    conv4_walk(reinterpret_cast<const f32x4*>(p.x) + c4, reinterpret_cast<const f32x4*>(p.state) + c4,
+               reinterpret_cast<const f32x4*>(p.w) + 4 * c4, reinterpret_cast<f32x4*>(o),
+               (size_t)p.conv_dim / 4, (size_t)row / 4, t0, min(p.n_tok, t0 + toks));
+}
+
+// Tokens a thread of the conv walks: 32, fewer where that leaves under 1024 workgroups (each
+// walk reads three rows more than it writes).
+int conv_toks(int32_t conv_dim, int32_t n_tok, int32_t n_seq) {
+    const long long bx = (conv_dim / 4 + 255) / 256 * (long long)n_seq;
+    int toks = 32;
+    while (toks > 4 && bx * ((n_tok + toks - 1) / toks) < 1024) toks /= 2;
+    return toks;
 }
 
 // New state = the last d_conv-1 rows of X_ext (after gdn_conv1d_kernel has
@@ -151,7 +204,7 @@ __global__ __launch_bounds__(256) void gdn_conv_state_shift_kernel(const float* 
 }
 
 // RMSNormGated (src/model/mod.rs:918-932) in place: for every (row, V head),
-// o * (1/sqrt(mean(o^2) + eps)) * w * silu(z).  One wavefront per (row, head).
+// o * (1/sqrt(mean(o^2) + eps)) * w * silu(z).  Any width: one wavefront per (row, head).
 __global__ __launch_bounds__(256) void gdn_rmsnorm_gated_kernel(float* __restrict__ o,
                                                                 const float* __restrict__ z,
                                                                 const float* __restrict__ w,
@@ -162,31 +215,6 @@ __global__ __launch_bounds__(256) void gdn_rmsnorm_gated_kernel(float* __restric
     if (hrow >= n_heads_total) return;
     float* oh = o + (size_t)hrow * v_hd;
     const float* zh = z + (size_t)hrow * v_hd;
-    if ((v_hd == 128 || v_hd == 64) && (((uintptr_t)oh | (uintptr_t)zh) & 7) == 0) {  // 8-byte accesses (v_hd 128)
-        typedef float f2 __attribute__((ext_vector_type(2)));
-        const int npl = v_hd / 64;  // values per lane: 2 (one f2) or 1
-        float ov[2] = {0.f, 0.f}, zv[2] = {0.f, 0.f};
-        if (npl == 2) {
-            const f2 a = reinterpret_cast<const f2*>(oh)[lane], b = reinterpret_cast<const f2*>(zh)[lane];
-            ov[0] = a[0]; ov[1] = a[1]; zv[0] = b[0]; zv[1] = b[1];
-        } else {
-            ov[0] = oh[lane];
-            zv[0] = zh[lane];
-        }
-        float sq = ov[0] * ov[0] + ov[1] * ov[1];
-#pragma unroll
-        for (int m = 32; m >= 1; m >>= 1) sq = wave_sum_xor(sq, m);
-        const float sc = 1.0f / sqrtf(sq / (float)v_hd + eps);
-        float r[2];
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const int d = npl * lane + e;
-            r[e] = e < npl ? (ov[e] * sc * w[d]) * (zv[e] / (1.0f + expf(-zv[e]))) : 0.f;
-        }
-        if (npl == 2) reinterpret_cast<f2*>(oh)[lane] = f2{r[0], r[1]};
-        else oh[lane] = r[0];
-        return;
-    }
     float ss = 0.f;
     for (int d = lane; d < v_hd; d += 64) ss += oh[d] * oh[d];
 #pragma unroll
@@ -195,6 +223,42 @@ __global__ __launch_bounds__(256) void gdn_rmsnorm_gated_kernel(float* __restric
     for (int d = lane; d < v_hd; d += 64) {
         const float zv = zh[d];
         oh[d] = (oh[d] * scale * w[d]) * (zv / (1.0f + expf(-zv)));
+    }
+}
+
+// The same at V = 64, 128 or 256 and 16-byte aligned rows: V / 4 lanes a row, so a wavefront
+// loads 256 / V rows with one 16-byte access per lane, and each wavefront takes NR such
+// groups, all requested before any is used: 4096 tokens x 32 heads x 128 (201 MB) in 31 us
+// (6.5 TB/s; 47 with one row and 8 bytes a lane per wavefront).
+template <int V>
+__global__ __launch_bounds__(256) void gdn_rmsnorm_gated_vec_kernel(float* __restrict__ o,
+                                                                    const float* __restrict__ z,
+                                                                    const float* __restrict__ w,
+                                                                    int n_rows, float eps) {
+    constexpr int LPR = V / 4, NR = 2;
+    const int lane = threadIdx.x & 63, c = 4 * (lane % LPR);
+    const int first = ((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6)) * NR * (64 / LPR) + lane / LPR;
+    f32x4 ov[NR], zv[NR];
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+        const size_t at = (size_t)min(first + i * (64 / LPR), n_rows - 1) * V + c;
+        ov[i] = *reinterpret_cast<const f32x4*>(o + at);
+        zv[i] = *reinterpret_cast<const f32x4*>(z + at);
+    }
+    const f32x4 wv = *reinterpret_cast<const f32x4*>(w + c);
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+        const int row = first + i * (64 / LPR);
+        float ss = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ss += ov[i][e] * ov[i][e];
+#pragma unroll
+        for (int m = LPR / 2; m >= 1; m >>= 1) ss = wave_sum_xor(ss, m);
+        const float scale = 1.0f / sqrtf(ss / (float)V + eps);
+        f32x4 r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[e] = (ov[i][e] * scale * wv[e]) * (zv[i][e] / (1.0f + expf(-zv[i][e])));
+        if (row < n_rows) *reinterpret_cast<f32x4*>(o + (size_t)row * V + c) = r;
     }
 }
 
@@ -685,6 +749,27 @@ __device__ __forceinline__ f32x4 mm16(const float* X, int xs, const float* Y, in
     return acc;
 }
 
+// The conv state's update, new state = the last three rows of X_ext, one thread per channel
+// (each reads all its rows before it writes any): done by the prep kernel of a layer prompt,
+// after the conv has read the old state and before the scan writes the caller's output.
+struct GdnConvRoll {
+    const float* x;
+    float* state;  // null: no update
+    int n_tok, conv_dim;
+};
+__device__ __forceinline__ void conv_roll(const GdnConvRoll& r, int wg, int n_wg) {
+    for (int i = wg * (int)blockDim.x + (int)threadIdx.x; i < r.conv_dim; i += n_wg * (int)blockDim.x) {
+        float v[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const int e = r.n_tok + j;  // X_ext row that becomes state row j
+            v[j] = e < 3 ? r.state[(size_t)e * r.conv_dim + i] : r.x[(size_t)(e - 3) * r.conv_dim + i];
+        }
+#pragma unroll
+        for (int j = 0; j < 3; ++j) r.state[(size_t)j * r.conv_dim + i] = v[j];
+    }
+}
+
 struct GdnWs {
     f16* q16;   // [n_chunks][Hk][64][128] q / max(|q|,1e-12) / sqrt(Dk), f16
     f16* k16;   // [n_chunks][Hk][64][128] k / max(|k|,1e-12), f16
@@ -706,7 +791,7 @@ __global__ __launch_bounds__(512) void gdn_prep_kernel(const float* __restrict__
                                                        const float* __restrict__ k,
                                                        const float* __restrict__ beta,
                                                        const float* __restrict__ g, int n_tok,
-                                                       int hk, int hv, GdnWs w) {
+                                                       int hk, int hv, GdnWs w, GdnConvRoll roll) {
     constexpr int BIG = 2 * PREP_B > 2 * GC * KS_ ? 2 * PREP_B : 2 * GC * KS_;
     __shared__ __attribute__((aligned(16))) float s_big[BIG];   // sk | sq, then 2 x (sa | st | sx)
     __shared__ __attribute__((aligned(16))) float skk[GC * TS_];  // K K^T (lower tiles)
@@ -719,6 +804,7 @@ __global__ __launch_bounds__(512) void gdn_prep_kernel(const float* __restrict__
     f16* sqh = skl + GC * KH_;
     f16* sql = sqh + GC * KH_;
     static_assert(4 * GC * KH_ * 2 <= BIG * 4, "phase A tiles fit s_big");
+    if (roll.state) conv_roll(roll, blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
     const int kh = blockIdx.y;
     const int n_chunks = (n_tok + GC - 1) / GC;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1300,11 +1386,12 @@ hipError_t launch_gdn_conv1d(const float* x, float* state, const float* w, float
     const size_t total = (size_t)n_seq * n_tok * conv_dim;
     const bool aligned =
         (((uintptr_t)x | (uintptr_t)state | (uintptr_t)w | (uintptr_t)out) & 15) == 0;
+    const int toks = conv_toks(conv_dim, n_tok, n_seq);
     if (d_conv == 4 && conv_dim % 4 == 0 && aligned && n_seq <= 65535)
         hipLaunchKernelGGL(gdn_conv1d_k4_kernel,
-                           dim3((unsigned)((conv_dim / 4 + 255) / 256), (unsigned)((n_tok + kConvTok - 1) / kConvTok),
+                           dim3((unsigned)((conv_dim / 4 + 255) / 256), (unsigned)((n_tok + toks - 1) / toks),
                                 (unsigned)n_seq),
-                           dim3(256), 0, s, x, state, w, out, n_tok, conv_dim);
+                           dim3(256), 0, s, x, state, w, out, n_tok, conv_dim, toks);
     else
         hipLaunchKernelGGL(gdn_conv1d_kernel, dim3(grid_of(total)), dim3(256), 0, s, x, state, w,
                            out, n_seq, n_tok, conv_dim, d_conv);
@@ -1319,9 +1406,55 @@ hipError_t launch_gdn_conv1d(const float* x, float* state, const float* w, float
     return hipGetLastError();
 }
 
+bool gdn_layer_in_ok(const float* x, const float* state, int32_t n_k_heads, int32_t n_v_heads,
+                     int32_t k_hd, int32_t v_hd, int32_t d_conv) {
+    return d_conv == 4 && (long long)n_k_heads * k_hd % 4 == 0 && (long long)n_v_heads * v_hd % 4 == 0 &&
+           (((uintptr_t)x | (uintptr_t)state) & 15) == 0;
+}
+
+hipError_t launch_gdn_layer_in(const float* x, const float* state, const float* w, const float* beta_raw,
+                               const float* a_raw, const float* ssm_a, const float* dt_bias, float* q,
+                               float* k, float* v, float* beta, float* g, int32_t n_tok,
+                               int32_t n_k_heads, int32_t n_v_heads, int32_t k_hd, int32_t v_hd,
+                               hipStream_t s) {
+    GdnLayerIn p{x, state, w, beta_raw, a_raw, ssm_a, dt_bias, q, k, v, beta, g};
+    p.n_tok = n_tok;
+    p.kd = n_k_heads * k_hd;
+    p.vd = n_v_heads * v_hd;
+    p.conv_dim = 2 * p.kd + p.vd;
+    p.hv = n_v_heads;
+    const int toks = conv_toks(p.conv_dim, n_tok, 1);
+    const int gx = (p.conv_dim / 4 + 255) / 256, ny = (n_tok + toks - 1) / toks;
+    // a few elements a thread for the gates
+    const long long gates = (long long)n_tok * n_v_heads;
+    const int ng = (int)std::max<long long>(1, std::min<long long>(1024, gates / (256LL * gx)));
+    hipLaunchKernelGGL(gdn_layer_in_kernel, dim3((unsigned)gx, (unsigned)(ny + ng)), dim3(256), 0, s, p, toks, ny);
+    return hipGetLastError();
+}
+
+hipError_t launch_gdn_conv_state(const float* x, float* state, int32_t n_tok, int32_t conv_dim, int32_t d_conv,
+                                 hipStream_t s) {
+    if (d_conv < 2) return hipSuccess;
+    if (n_tok >= d_conv - 1)
+        hipLaunchKernelGGL(gdn_conv_state_kernel, dim3(grid_of((size_t)(d_conv - 1) * conv_dim)),
+                           dim3(256), 0, s, x, state, 1, n_tok, conv_dim, d_conv);
+    else
+        hipLaunchKernelGGL(gdn_conv_state_shift_kernel, dim3(grid_of((size_t)conv_dim)),
+                           dim3(256), 0, s, x, state, 1, n_tok, conv_dim, d_conv);
+    return hipGetLastError();
+}
+
 hipError_t launch_gdn_rmsnorm_gated(float* o, const float* z, const float* w, int32_t n_rows,
                                     int32_t n_v_heads, int32_t v_hd, float eps, hipStream_t s) {
     const int n = n_rows * n_v_heads;
+    if ((v_hd == 64 || v_hd == 128 || v_hd == 256) && (((uintptr_t)o | (uintptr_t)z | (uintptr_t)w) & 15) == 0) {
+        const int per = 4 * 2 * (256 / v_hd);  // rows a workgroup
+        const dim3 grid((unsigned)((n + per - 1) / per));
+        if (v_hd == 64) hipLaunchKernelGGL(gdn_rmsnorm_gated_vec_kernel<64>, grid, dim3(256), 0, s, o, z, w, n, eps);
+        else if (v_hd == 128) hipLaunchKernelGGL(gdn_rmsnorm_gated_vec_kernel<128>, grid, dim3(256), 0, s, o, z, w, n, eps);
+        else hipLaunchKernelGGL(gdn_rmsnorm_gated_vec_kernel<256>, grid, dim3(256), 0, s, o, z, w, n, eps);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(gdn_rmsnorm_gated_kernel, dim3((n + 3) / 4), dim3(256), 0, s, o, z, w, n,
                        v_hd, eps);
     return hipGetLastError();
@@ -1401,7 +1534,8 @@ size_t gdn_prefill_ws_floats(int32_t n_tok, int32_t n_k_heads, int32_t n_v_heads
 hipError_t launch_gdn_prefill(const float* q, const float* k, const float* v, const float* beta,
                               const float* g, float* state, float* out, int32_t n_tok,
                               int32_t n_k_heads, int32_t n_v_heads, int32_t chunk,
-                              const GdnWorkspace& ws, hipStream_t s) {
+                              const GdnWorkspace& ws, hipStream_t s, const float* conv_x,
+                              float* conv_state, int32_t conv_dim) {
     if (chunk != GC) return hipErrorInvalidValue;
     if (n_tok <= 0) return hipSuccess;  // the kernels clamp token indices to n_tok - 1
     const size_t nc = (size_t)(n_tok + GC - 1) / GC;
@@ -1419,7 +1553,7 @@ hipError_t launch_gdn_prefill(const float* q, const float* k, const float* v, co
     if (e0 != hipSuccess) return e0;
     const unsigned gx = (unsigned)std::max<size_t>(1, std::min<size_t>(nc, (size_t)n_cu / n_k_heads));
     hipLaunchKernelGGL(gdn_prep_kernel, dim3(gx, n_k_heads), dim3(512), 0, s, q, k, beta, g,
-                       n_tok, n_k_heads, n_v_heads, w);
+                       n_tok, n_k_heads, n_v_heads, w, GdnConvRoll{conv_x, conv_state, n_tok, conv_dim});
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(gdn_scan_kernel, dim3(n_v_heads * (DV / SCOLS)), dim3(768), 0, s, q, k, v,

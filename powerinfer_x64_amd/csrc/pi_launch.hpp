@@ -202,6 +202,20 @@ hipError_t launch_gdn_gates(const float* beta_raw, const float* a_raw, const flo
 hipError_t launch_gdn_conv1d(const float* x, float* state, const float* w, float* out,
                              int32_t n_seq, int32_t n_tok, int32_t conv_dim, int32_t d_conv,
                              hipStream_t s);
+// A layer step's conv1d + SiLU over its q | k | v channels and its gates in one launch, the conv
+// split into q, k [n_tok][n_k_heads k_hd] and v [n_tok][n_v_heads v_hd]; the conv state is
+// read, its update is launch_gdn_prefill's (k_hd = v_hd = 128) or launch_gdn_conv_state's.
+// For d_conv 4, widths that are multiples of 4 and 16-byte aligned x and state
+// (gdn_layer_in_ok; q, k, v, w aligned too).
+bool gdn_layer_in_ok(const float* x, const float* state, int32_t n_k_heads, int32_t n_v_heads,
+                     int32_t k_hd, int32_t v_hd, int32_t d_conv);
+hipError_t launch_gdn_layer_in(const float* x, const float* state, const float* w, const float* beta_raw,
+                               const float* a_raw, const float* ssm_a, const float* dt_bias, float* q,
+                               float* k, float* v, float* beta, float* g, int32_t n_tok,
+                               int32_t n_k_heads, int32_t n_v_heads, int32_t k_hd, int32_t v_hd,
+                               hipStream_t s);
+hipError_t launch_gdn_conv_state(const float* x, float* state, int32_t n_tok, int32_t conv_dim, int32_t d_conv,
+                                 hipStream_t s);
 hipError_t launch_gdn_rmsnorm_gated(float* o, const float* z, const float* w, int32_t n_rows,
                                     int32_t n_v_heads, int32_t v_hd, float eps, hipStream_t s);
 // One GDN layer step of one token, k_hd = v_hd = 128, d_conv 4: conv1d + SiLU
@@ -241,9 +255,12 @@ struct GdnWorkspace {
     size_t capacity;  // floats
 };
 size_t gdn_prefill_ws_floats(int32_t n_tok, int32_t n_k_heads, int32_t n_v_heads, int32_t chunk);
+// conv_state (optional): also rolled by n_tok rows of conv_x, [3][conv_dim] (d_conv 4), before
+// anything is written to out.
 hipError_t launch_gdn_prefill(const float* q, const float* k, const float* v, const float* beta,
                               const float* g, float* state, float* out, int32_t n_tok,
                               int32_t n_k_heads, int32_t n_v_heads, int32_t chunk,
-                              const GdnWorkspace& ws, hipStream_t s);
+                              const GdnWorkspace& ws, hipStream_t s, const float* conv_x = nullptr,
+                              float* conv_state = nullptr, int32_t conv_dim = 0);
 
 }  // namespace pi

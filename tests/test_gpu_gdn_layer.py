@@ -5,9 +5,10 @@ RMSNormGated, with both states carried across calls and cleared by reset
 (src/model/mod.rs:1867-1869)."""
 import numpy as np
 import pytest
+import torch
 
 from oracle import oracle as orc
-from tests.gpu_util import device
+from tests.gpu_util import device, to_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -182,3 +183,32 @@ def test_gdn_layer_reset_orders_after_side_stream_steps():
         assert np.array_equal(g.cpu().numpy().view(np.uint32), want.view(np.uint32))
     used.close()
     fresh.close()
+
+
+@pytest.mark.parametrize("hk,hv,dk,dv", [(2, 4, 128, 128), (1, 2, 64, 32)])
+@pytest.mark.parametrize("lens", [(2, 3), (3, 2, 5), (31, 33), (64, 130, 2)])
+def test_layer_prompts_equal_the_separate_steps(hk, hv, dk, dv, lens):
+    """A layer prompt's fused launches (conv split into q, k, v beside the gates; the conv state
+    rolled by the recurrence's first kernel) against the public steps one by one, over calls that
+    continue each other with fewer, as many and more tokens than the conv state holds: the same
+    kernels' arithmetic, so bit for bit.  The second time the output overwrites the conv input."""
+    from powerinfer_x64_amd import runtime as rt
+    dev = device()
+    rng = np.random.default_rng(sum(lens) + dk)
+    conv = 2 * hk * dk + hv * dv
+    f = lambda *s: rng.standard_normal(s).astype(np.float32)  # noqa: E731
+    w, a, dt, nw = f(conv, 4) * 0.5, -np.abs(f(hv)), f(hv) * 0.1, rng.uniform(0.5, 1.5, dv).astype(np.float32)
+    layers = [rt.GdnLayer(dev, hk, hv, dk, dv, w, a, dt, nw, 1e-6) for _ in range(2)]
+    cs, st = torch.zeros((1, 3, conv), device="cuda"), torch.zeros((hv, dk, dv), device="cuda")
+    for n in lens:
+        x, z, br, ar = (to_dev(f(*s)) for s in ((n, conv), (n, hv, dv), (n, hv), (n, hv)))
+        act = rt.gdn_conv1d(dev, x[None], cs, to_dev(w))[0]
+        q, k, v = (t.contiguous().view(n, h, d) for t, h, d in zip(
+            act.split([hk * dk, hk * dk, hv * dv], dim=1), (hk, hk, hv), (dk, dk, dv)))
+        beta, g = rt.gdn_gates(dev, br, ar, to_dev(a), to_dev(dt))
+        ref = rt.gdn_prefill(dev, q, k, v, beta, g, st)
+        rt.gdn_rmsnorm_gated(dev, ref, z, to_dev(nw), 1e-6)
+        assert torch.equal(layers[0].forward_dev(x, z, br, ar), ref)
+        buf = x.reshape(-1)
+        out = layers[1].forward_dev(x, z, br, ar, buf[:n * hv * dv].view(n, hv, dv))
+        assert torch.equal(out, ref)
