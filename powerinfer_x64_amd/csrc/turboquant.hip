@@ -15,8 +15,7 @@
 // file is built with -ffp-contract=off), sqrt and divide are correctly
 // rounded, the nearest
 // centroid takes the first strict minimum, and a QJL bit is set for a
-// projection >= 0.  One wavefront per (sequence, token, KV
-// head); lane i owns rotated coordinates i + 64 j, j < D / 64.
+// projection >= 0.
 #include "pi_device.hpp"
 #include "pi_launch.hpp"
 
@@ -60,109 +59,203 @@ __device__ __forceinline__ int nearest_centroid(float x) {
     return best;
 }
 
-template <int D>
+// Bit i of the 12-bit x to bit 3 i.
+__device__ __forceinline__ uint64_t spread3(uint32_t x) {
+    x &= 0xfffu;
+    x = (x | x << 16) & 0x0f0000ffu;
+    x = (x | x << 8) & 0x0f00f00fu;
+    x = (x | x << 4) & 0xc30c30c3u;
+    return ((uint64_t)x | (uint64_t)x << 2) & 0x249249249ull;
+}
+
+// A group of R tokens of one KV head: positions gp .. gp + R - 1, gp a multiple of R (so they
+// share a page), those of them that the launch covers.  WPR wavefronts share a group: lane l
+// of wavefront i owns rotated coordinates 64 (i D / 64 / WPR + j) + l of every row.
+//
+// What bounds it: each row is 2 D multiply-and-adds per coordinate that may not fuse (27 us
+// of vector instructions for 16 384 rows of 128), so the matrices must not cost as much as
+// that: one wavefront per row read 2 D D values a row through the L1 (87 us).  With R rows a
+// matrix value is loaded once for R rows, some columns ahead of its use, and the rows'
+// values come from LDS as 16-byte broadcasts; few rows are bound by the chain of column loads,
+// so their coordinates spread over more wavefronts and more columns are in flight.  The
+// sequential norms of the R rows run in R lanes side by side, the codes are packed from
+// ballots (three masks of 64 coordinates make six dwords) in one lane per row and 64
+// coordinates, and R tokens of a value dim are one store.
+template <int D, int R, int WPR>
 __global__ __launch_bounds__(256) void tq_append_kernel(TqPool t, const float* __restrict__ k,
                                                         const float* __restrict__ v,
                                                         const int32_t* __restrict__ page_table,
                                                         int max_pages,
                                                         const int32_t* __restrict__ start_pos,
-                                                        int n_seq, int n_tok) {
-    constexpr int NJ = D / 64;          // coordinates per lane
+                                                        int n_seq, int n_tok, int n_grp) {
+    constexpr int NJ = D / 64 / WPR;    // coordinates per lane
+    constexpr int CF = R == 1 ? 16 : R == 2 ? 8 : 4;  // matrix columns requested at a time
     constexpr int CW = 3 * D / 32;      // record dwords of the 3-bit codes
     constexpr int KB = tq_key_bytes(D);
-    __shared__ float s_x[4][D];
-    __shared__ uint32_t s_bits[4][CW];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    constexpr int XS = D + 4;           // row stride: R rows' 16-byte reads on distinct banks
+    constexpr int GPW = 4 / WPR;        // row groups per workgroup
+    __shared__ __attribute__((aligned(16))) float s_x[GPW][R * XS];
+    const int lane = threadIdx.x & 63, w = (int)(threadIdx.x >> 6) / WPR;
+    const int j0 = (int)(threadIdx.x >> 6) % WPR * NJ;  // this wavefront's coordinates: 64 (j0 + j) + lane
     const int n_kv = t.g.n_kv_heads;
-    const long long item = (long long)blockIdx.x * 4 + w;
-    const bool on = item < (long long)n_seq * n_tok * n_kv;
-    const long long it = on ? item : 0;
-    const int kvh = (int)(it % n_kv);
-    const int tok = (int)((it / n_kv) % n_tok);
-    const int seq = (int)(it / ((long long)n_kv * n_tok));
-    const size_t row = (((size_t)seq * n_tok + tok) * n_kv + kvh) * D;
+    // group (head, sequence, positions), the head slowest: a workgroup's wavefronts share its matrices
+    const long long item = (long long)blockIdx.x * GPW + w, items = (long long)n_kv * n_seq * n_grp;
+    const long long it = item < items ? item : items - 1;
+    const int kvh = (int)(it / ((long long)n_seq * n_grp));
+    const int seq = (int)(it / n_grp % n_seq);
+    const int start = start_pos[seq];
+    const long long gp = (long long)(start & ~(R - 1)) + (it % n_grp) * R;
+    auto tok_of = [&](int r) { return (int)min(max(gp + r - start, 0LL), (long long)n_tok - 1); };
+    auto row_of = [&](int r) { return (((size_t)seq * n_tok + tok_of(r)) * n_kv + kvh) * D; };
+    float* sx = s_x[w];
 
-    // L2 norm: sequential f32 sum of squares (:466-468)
+    // L2 norms: sequential f32 sums of squares (:466-468), row r in lanes r, r + R, ..
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) s_x[w][lane + 64 * j] = k[row + lane + 64 * j];
-    if (lane < CW) s_bits[w][lane] = 0u;
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) sx[r * XS + lane + 64 * (j0 + j)] = k[row_of(r) + lane + 64 * (j0 + j)];
     __syncthreads();
     float ss = 0.f;
-    for (int j = 0; j < D; ++j) ss = __fadd_rn(ss, __fmul_rn(s_x[w][j], s_x[w][j]));
+    {
+        const f32x4* xr = reinterpret_cast<const f32x4*>(sx + (lane % R) * XS);
+#pragma unroll 4
+        for (int i = 0; i < D / 4; ++i) {
+            const f32x4 x = xr[i];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ss = __fadd_rn(ss, __fmul_rn(x[e], x[e]));
+        }
+    }
     const float norm = sqrt_rn(ss);
     const float inv = norm > 1e-12f ? __fdiv_rn(1.0f, norm) : 0.0f;
-    float x[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) x[j] = __fmul_rn(s_x[w][lane + 64 * j], inv);
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) s_x[w][lane + 64 * j] = x[j];
+    for (int r = 0; r < R; ++r) {
+        const float ir = __shfl(inv, r, 64);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            float* x = sx + r * XS + lane + 64 * (j0 + j);
+            *x = __fmul_rn(*x, ir);
+        }
+    }
     __syncthreads();
 
-    // rotation rows lane + 64 j, then the sqrt(d) scale (:131-146)
-    const float* rt = t.rt + (size_t)kvh * D * D;
-    float r[NJ];
+    // acc[r][j] = row lane + 64 j of the (transposed) matrix times row r, in column order
+    auto product = [&](const float* m, float (&acc)[R][NJ]) {
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) r[j] = 0.f;
-    for (int i = 0; i < D; ++i) {
-        const float xi = s_x[w][i];
+        for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) r[j] = __fadd_rn(r[j], __fmul_rn(rt[i * D + lane + 64 * j], xi));
-    }
-    int c[NJ];
+            for (int j = 0; j < NJ; ++j) acc[r][j] = 0.f;
+        float m0[CF][NJ], m1[CF][NJ];
+        auto fetch = [&](int i, float (&d)[CF][NJ]) {
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-        r[j] = __fmul_rn(r[j], t.scale);
-        c[j] = nearest_centroid(r[j]);
-    }
+            for (int e = 0; e < CF; ++e)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) d[e][j] = m[(i + e) * D + lane + 64 * (j0 + j)];
+            __builtin_amdgcn_sched_barrier(0);  // requested here, ahead of the columns in hand
+        };
+        auto add = [&](int i, const float (&d)[CF][NJ]) {
+#pragma unroll
+            for (int c = 0; c < CF; c += 4)
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const f32x4 x = *reinterpret_cast<const f32x4*>(sx + r * XS + i + c);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j) acc[r][j] = __fadd_rn(acc[r][j], __fmul_rn(d[c + e][j], x[e]));
+                }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        fetch(0, m0);
+        for (int i = 0; i < D; i += 2 * CF) {
+            fetch(i + CF, m1);
+            add(i, m0);
+            fetch(min(i + 2 * CF, D - CF), m0);
+            add(i + CF, m1);
+        }
+    };
+
+    // rotation rows lane + 64 j, then the sqrt(d) scale (:131-146); the codes' bit masks and
+    // the residual (:170-173).  Lane r NJ + j keeps the masks of row r, coordinates 64 j ..
+    float acc[R][NJ];
+    product(t.rt + (size_t)kvh * D * D, acc);
     __syncthreads();
-    // residual (:170-173); codes: coordinate i occupies bits 3i .. 3i+2 of the record
+    uint32_t mk[3][2] = {};  // code bits 0..2 of the lane's 64 coordinates
+    auto keep = [&](uint32_t (&dst)[2], uint64_t m, int at) {
+        dst[0] = lane == at ? (uint32_t)m : dst[0];
+        dst[1] = lane == at ? (uint32_t)(m >> 32) : dst[1];
+    };
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-        const int i = lane + 64 * j;
-        s_x[w][i] = __fsub_rn(r[j], kCentroids3[c[j]]);
-        const uint32_t cv = (uint32_t)c[j];
-        const int bit = 3 * i, wd = bit >> 5, off = bit & 31;
-        atomicOr(&s_bits[w][wd], cv << off);
-        if (off > 29) atomicOr(&s_bits[w][wd + 1], cv >> (32 - off));
-    }
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const float x = __fmul_rn(acc[r][j], t.scale);
+            const int c = nearest_centroid(x);
+            sx[r * XS + lane + 64 * (j0 + j)] = __fsub_rn(x, kCentroids3[c]);
+#pragma unroll
+            for (int b = 0; b < 3; ++b) keep(mk[b], __ballot(c >> b & 1), r * NJ + j);
+        }
     __syncthreads();
 
     // QJL signs of G . residual (:176-184), one ballot per 64 projections
-    const float* gt = t.gt + (size_t)kvh * D * D;
-    float pr[NJ];
+    product(t.gt + (size_t)kvh * D * D, acc);
+    uint32_t sg[2] = {};
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) pr[j] = 0.f;
-    for (int i = 0; i < D; ++i) {
-        const float ri = s_x[w][i];
+    for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) pr[j] = __fadd_rn(pr[j], __fmul_rn(gt[i * D + lane + 64 * j], ri));
-    }
-    uint64_t m[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) m[j] = __ballot(pr[j] >= 0.0f);
-    if (!on) return;
+        for (int j = 0; j < NJ; ++j) keep(sg, __ballot(acc[r][j] >= 0.0f), r * NJ + j);
 
-    const int pos = start_pos[seq] + tok;
-    if (pos < 0 || pos / kPageTokens >= max_pages) return;  // outside the sequence's table
-    const int page = page_table[(size_t)seq * max_pages + pos / kPageTokens];
+    // outside the sequence's table or the pool: nothing is stored
+    if (item >= items || gp < 0 || gp / kPageTokens >= max_pages) return;
+    const int page = page_table[(size_t)seq * max_pages + gp / kPageTokens];
     if (page < 0 || page >= t.g.n_pages) return;
-    const int slot = pos % kPageTokens;
+    const int s0 = (int)(gp % kPageTokens);
+    auto live = [&](int r) { return gp + r >= start && gp + r < (long long)start + n_tok; };
     const size_t blk = (size_t)page * n_kv + kvh;
     char* kb = reinterpret_cast<char*>(t.g.k) + blk * (kPageTokens * (KB + 4));
-    uint32_t* rec = reinterpret_cast<uint32_t*>(kb + slot * KB);
-    if (lane < CW) rec[lane] = s_bits[w][lane];
+    if (lane < R * NJ && live(lane / NJ)) {
+        const int r = lane / NJ, j = j0 + lane % NJ;
+        uint32_t* rec = reinterpret_cast<uint32_t*>(kb + (s0 + r) * KB);
+        const uint64_t b0 = (uint64_t)mk[0][1] << 32 | mk[0][0], b1 = (uint64_t)mk[1][1] << 32 | mk[1][0],
+                       b2 = (uint64_t)mk[2][1] << 32 | mk[2][0];
+        // coordinate i occupies bits 3i .. 3i+2 of the record: dword d of the 64 coordinates
+        // starts 32 d - 3 i0 bits into coordinate i0 = 32 d / 3
+#pragma unroll
+        for (int d = 0; d < 6; ++d) {
+            const int i0 = 32 * d / 3;
+            const uint64_t code = spread3((uint32_t)(b0 >> i0)) | spread3((uint32_t)(b1 >> i0)) << 1 |
+                                  spread3((uint32_t)(b2 >> i0)) << 2;
+            rec[6 * j + d] = (uint32_t)(code >> (32 * d - 3 * i0));
+        }
+        rec[CW + 2 * j] = sg[0];
+        rec[CW + 2 * j + 1] = sg[1];
+    }
+    if (j0 == 0 && lane < R && live(lane)) reinterpret_cast<float*>(kb + kPageTokens * KB)[s0 + lane] = norm;
+    // values as f16 (round to nearest even), V block [dim][16 tokens]
+    typedef f16 f16r __attribute__((ext_vector_type(R)));
+    f16* vb = reinterpret_cast<f16*>(t.g.v) + blk * (kPageTokens * D) + s0;
+    const bool whole = live(0) && live(R - 1);
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
-        if (lane == CW + 2 * j) rec[CW + 2 * j] = (uint32_t)m[j];
-        if (lane == CW + 2 * j + 1) rec[CW + 2 * j + 1] = (uint32_t)(m[j] >> 32);
-    }
-    if (lane == 63) reinterpret_cast<float*>(kb + kPageTokens * KB)[slot] = norm;
-    // values as f16 (round to nearest even), V block [dim][16 tokens]
-    f16* vb = reinterpret_cast<f16*>(t.g.v) + blk * (kPageTokens * D);
+        f16* vd = vb + (lane + 64 * (j0 + j)) * kPageTokens;
+        f16 x[R];
 #pragma unroll
-    for (int j = 0; j < NJ; ++j)
-        vb[(lane + 64 * j) * kPageTokens + slot] = to_f16(v[row + lane + 64 * j]);
+        for (int r = 0; r < R; ++r) x[r] = to_f16(v[row_of(r) + lane + 64 * (j0 + j)]);
+        if (whole) {
+            if constexpr (R == 1) {
+                vd[0] = x[0];
+            } else {
+                f16r o;
+#pragma unroll
+                for (int r = 0; r < R; ++r) o[r] = x[r];
+                *reinterpret_cast<f16r*>(vd) = o;
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (live(r)) vd[r] = x[r];
+        }
+    }
 }
 
 // Stored records of tokens start .. start+n_tok-1 of one sequence: keys
@@ -618,13 +711,40 @@ hipError_t launch_tq_append(const TqPool& t, const float* k, const float* v,
     if (items <= 0) return hipSuccess;
     if ((items + 3) / 4 > 0x7fffffffLL) return hipErrorInvalidValue;
     const dim3 grid((unsigned)((items + 3) / 4));
-    if (t.g.head_dim == 128)
-        hipLaunchKernelGGL(tq_append_kernel<128>, grid, dim3(256), 0, s, t, k, v, page_table, max_pages,
-                           start_pos, n_seq, n_tok);
-    else if (t.g.head_dim == 256)
-        hipLaunchKernelGGL(tq_append_kernel<256>, grid, dim3(256), 0, s, t, k, v, page_table, max_pages,
-                           start_pos, n_seq, n_tok);
-    else if (t.g.head_dim < 1 || t.g.head_dim > kTqMaxDim)
+    if (t.g.head_dim == 128 || t.g.head_dim == 256) {
+        // Rows a group (r): as many as leave the chip enough wavefronts.  A group's coordinates
+        // are split over D / 64 wavefronts, until the launch is so large that reading the rows'
+        // LDS values in each of them costs more than the shorter chains save.  Measured, D 128
+        // (8 heads): 8 rows 8.2 us (r 1), 2048 rows 13.8 (r 2; 16.2 at r 1), 8192 28.4 (r 4; 32.8
+        // at r 2), 16 384 44.5 (r 8; 46.5 at r 4), 131 072 212 (one wavefront a group; 231 split);
+        // D 256 (2 heads): 2 rows 12.6 (23.6 unsplit), 2048 33.9 (r 4), 32 768 236.
+        const long long units = items * (t.g.head_dim / 128);
+        const int r = units >= 8192 ? 8 : units >= 4096 ? 4 : units >= 2048 ? 2 : 1;
+        const int wpr = units >= 65536 ? 1 : t.g.head_dim / 64;
+        // groups of r aligned positions that n_tok positions from anywhere can touch
+        const long long n_grp = ((long long)n_tok + r - 2) / r + 1;
+        const long long waves = n_grp * n_seq * t.g.n_kv_heads * wpr;
+        if ((waves + 3) / 4 > 0x7fffffffLL || n_grp > 0x7fffffffLL) return hipErrorInvalidValue;
+        const dim3 gr((unsigned)((waves + 3) / 4));
+#define PI_TQ_APPEND(DD, RR, WW)                                                                            \
+    hipLaunchKernelGGL((tq_append_kernel<DD, RR, WW>), gr, dim3(256), 0, s, t, k, v, page_table, max_pages, \
+                       start_pos, n_seq, n_tok, (int)n_grp)
+#define PI_TQ_APPEND_D(DD)                                     \
+    if (wpr == 1) PI_TQ_APPEND(DD, 8, 1);                      \
+    else switch (r) {                                          \
+        case 8: PI_TQ_APPEND(DD, 8, DD / 64); break;           \
+        case 4: PI_TQ_APPEND(DD, 4, DD / 64); break;           \
+        case 2: PI_TQ_APPEND(DD, 2, DD / 64); break;           \
+        default: PI_TQ_APPEND(DD, 1, DD / 64);                 \
+    }
+        if (t.g.head_dim == 128) {
+            PI_TQ_APPEND_D(128)
+        } else {
+            PI_TQ_APPEND_D(256)
+        }
+#undef PI_TQ_APPEND_D
+#undef PI_TQ_APPEND
+    } else if (t.g.head_dim < 1 || t.g.head_dim > kTqMaxDim)
         return hipErrorInvalidValue;
     else {
 #define PI_TQ_ANY(NJ)                                                                              \

@@ -210,3 +210,28 @@ def test_decode_c4_shape_d256_gate(gqa_mode):
         err = row_rel_err(out[i], refs[i])
         print(f"\nD 256 seq {i} (L={lens[i]}): rel err {err:.3e}")
         assert err <= 1e-2, f"seq {i} (L={lens[i]}): rel err {err}"
+
+
+# groups of 1, 2, 4 and 8 tokens and unsplit groups of 8 (the row counts that pick each), starts
+# inside a group, several sequences a launch, and a launch that ends mid-group
+@pytest.mark.parametrize("d,hkv,n_tok", [(128, 2, 5), (128, 8, 270), (128, 8, 515), (128, 8, 1027), (256, 2, 515),
+                                         (256, 2, 1030), (256, 4, 1031), (128, 16, 4099), (256, 8, 4097)])
+def test_append_row_groups_bit_exact(d, hkv, n_tok):
+    dev = device()
+    rng = np.random.default_rng(d + n_tok)
+    starts = [3, 16] if n_tok < 1000 else [21]
+    R, G = _matrices(hkv, d)
+    pages = (max(starts) + n_tok + 15) // 16
+    pt = rng.permutation(len(starts) * pages).reshape(len(starts), pages).astype(np.int32)
+    k, v = (rng.standard_normal((len(starts), n_tok, hkv, d)).astype(np.float32) for _ in range(2))
+    pool = rt.TqPool(dev, pt.size, hkv, head_dim=d)
+    pool.append(to_dev(k), to_dev(v), to_dev(pt), to_dev(np.array(starts, np.int32)))
+    toks = sorted({0, 1, 4, min(7, n_tok - 1), n_tok - 2, n_tok - 1} | set(rng.integers(0, n_tok, 20).tolist()))
+    for i, s0 in enumerate(starts):
+        keys, norms, vals = (x.cpu().numpy() for x in pool.read(to_dev(pt), i, s0, n_tok))
+        if s0 % 16:  # the slots before the launch stay as the pool was created
+            assert not pool.read(to_dev(pt), i, 0, s0)[2].any()
+        assert np.array_equal(vals, v[i].astype(np.float16))
+        for t in toks:
+            want, wn = o.tq_cache_append_keys(k[i, t], R, G)
+            assert np.array_equal(keys[t], want[:, :keys.shape[-1]]) and np.array_equal(norms[t], wn)
