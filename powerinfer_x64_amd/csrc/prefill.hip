@@ -195,11 +195,15 @@ __global__ __launch_bounds__(64 * PrefillCfg<D>::NW, 1) void prefill_fa_kernel(P
             return;
     }
     const int nqb = (a.S + WROWS - 1) / WROWS;
-    const int by = blockIdx.y;
+    int by = blockIdx.y, bz = blockIdx.z;
+    if (!PG && a.ksplit == 1) {  // launch_d's grid order
+        by = blockIdx.z;
+        bz = blockIdx.y;
+    }
     const int n_blocks = a.paired && by != nqb - 1 - by ? 2 : 1;
     for (int blk = 0; blk < n_blocks; ++blk) {
     // heaviest (latest) query blocks first; a paired workgroup then takes block y
-    int qb = blk == 0 ? (a.paired ? nqb - 1 - by : (int)gridDim.y - 1 - by) : by;
+    int qb = blk == 0 ? (nqb - 1 - by) : by;
     if (blk > 0) {
         // every wave is past its last LDS read of the previous block before the
         // new block's loads land in the unit buffers
@@ -215,7 +219,7 @@ __global__ __launch_bounds__(64 * PrefillCfg<D>::NW, 1) void prefill_fa_kernel(P
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int hs = wave % HPW, rt = wave / HPW;
-    const int b = (int)blockIdx.z / a.ksplit, ksp = (int)blockIdx.z % a.ksplit;
+    const int b = bz / a.ksplit, ksp = bz % a.ksplit;
     const int S = a.S, Sk = a.Sk, q_off = a.q_off;
     const int per_kv = a.group / HPW;           // workgroups per KV head
     const int kvh = bxx / per_kv;
@@ -821,10 +825,14 @@ __global__ __launch_bounds__(512, 1) void prefill_fa256_kernel(PrefillArgs a) {
             return;
     }
     const int nqb = (a.S + WROWS - 1) / WROWS;
-    const int by = blockIdx.y;
+    int by = blockIdx.y, bz = blockIdx.z;
+    if (!PG && a.ksplit == 1) {  // launch_d's grid order
+        by = blockIdx.z;
+        bz = blockIdx.y;
+    }
     const int n_blocks = a.paired && by != nqb - 1 - by ? 2 : 1;
     for (int blk = 0; blk < n_blocks; ++blk) {
-    int qb = blk == 0 ? (a.paired ? nqb - 1 - by : (int)gridDim.y - 1 - by) : by;
+    int qb = blk == 0 ? (nqb - 1 - by) : by;
     if (blk > 0) {  // the previous block's LDS reads are done before new loads land
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
@@ -836,7 +844,7 @@ __global__ __launch_bounds__(512, 1) void prefill_fa256_kernel(PrefillArgs a) {
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int hs = wave % HPW, rt = wave / HPW;
-    const int b = (int)blockIdx.z / a.ksplit, ksp = (int)blockIdx.z % a.ksplit;
+    const int b = bz / a.ksplit, ksp = bz % a.ksplit;
     const int S = a.S, Sk = a.Sk, q_off = a.q_off;
     const int per_kv = a.group / HPW;
     const int kvh = bxx / per_kv;
@@ -1854,12 +1862,16 @@ template <int D>
 void launch_d(const PrefillArgs& a, int hpw, int n_kv_heads, int seq_len, int batch, bool bf,
               hipStream_t s) {
     constexpr int NW = PrefillCfg<D>::NW;
-    // x = workgroup's head set (fastest), y = query block (reversed in the
-    // kernel so the heaviest blocks go first); with x = KV head and
+    // x = workgroup's head set (fastest), y = sequence, z = query block (reversed in the
+    // kernel, so the heaviest blocks of all sequences go first: 4 prompts of 777 tokens,
+    // 32/8 heads, D 64 39.6 -> 33.2 us against the sequence slowest); with x = KV head and
     // round-robin dispatch over the 8 XCDs, a KV head's K/V stays in one L2.
+    // A key split keeps y = query block, z = (sequence, split): the splits of a block
+    // next to each other ran 1000 tokens at D 128 in 40.5 us instead of 33.9.
     const int rows = ROWS * NW / hpw;
     const int nqb = (seq_len + rows - 1) / rows;
-    const dim3 grid(n_kv_heads * (a.group / hpw), a.paired ? (nqb + 1) / 2 : nqb, batch * a.ksplit);
+    const unsigned gx = n_kv_heads * (a.group / hpw), blocks = a.paired ? (nqb + 1) / 2 : nqb;
+    const dim3 grid = a.ksplit > 1 ? dim3(gx, blocks, batch * a.ksplit) : dim3(gx, batch, blocks);
     const dim3 block(64 * NW);
     if constexpr (D == 256) {
         if (use_fa256()) {  // same grid: 128 / hpw query rows per workgroup either way
@@ -1915,7 +1927,7 @@ struct PrefillSched {
 };
 
 // The schedule of a launch.  Causal launches whose pairs of query blocks fill every CU
-// once or more pair them (equal work per workgroup).  Otherwise, a launch with fewer
+// in whole rounds pair them (equal work per workgroup).  Otherwise, a launch with fewer
 // workgroups than CUs may split a workgroup's keys over up to 4 workgroups (more CUs
 // busy, one merge launch after); ksplit is the number of partial slots the workspace
 // holds, split_plan picks the pieces.  PI_PREFILL_PAIRED=0 / 1 and PI_PREFILL_KSPLIT=n
@@ -1932,7 +1944,12 @@ PrefillSched prefill_sched(int batch, int seq_len, int n_q_heads, int n_kv_heads
     const long long pairs = (long long)n_kv_heads * (group / sc.hpw) * batch *
                             (((seq_len + rows - 1) / rows + 1) / 2);
     const int n_cu = cu_count();
-    sc.paired = causal && n_cu > 0 && pairs >= n_cu;
+    // Paired workgroups run in rounds of one per CU, so a last round that leaves CUs idle costs
+    // a whole pair: 3 prompts of 1500 tokens (288 pairs), 32/8 heads D 128 111 us against 81 in
+    // single blocks, heaviest first; 5000 tokens (320 pairs) 278 against 215.  With full rounds
+    // pairing is 1-3 % faster (4096 tokens, 256 pairs: 139.4 against 140.8).
+    const long long rounds = n_cu > 0 ? (pairs + n_cu - 1) / n_cu : 0;
+    sc.paired = causal && n_cu > 0 && pairs >= n_cu && 20 * pairs >= 19 * rounds * n_cu;
     const char* env_p = std::getenv("PI_PREFILL_PAIRED");  // read per call, as is PI_PREFILL_KSPLIT
     if (env_p && causal) sc.paired = env_p[0] == '1';
     sc.ksplit = 1;

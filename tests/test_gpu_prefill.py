@@ -14,7 +14,7 @@ import torch
 
 from oracle import oracle as orc
 from tests import ref64
-from tests.gpu_util import argmax_agreement, device, row_rel_err
+from tests.gpu_util import argmax_agreement, device, row_rel_err, to_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -286,3 +286,20 @@ def test_prefill_running_max_moves_in_late_tiles(s, hq, hkv, d):
     ref = _oracle_rows(tq, tk, tv, range(s))
     assert np.isfinite(out).all()
     assert row_rel_err(out, ref) <= 1e-2
+
+
+@pytest.mark.parametrize("paired", ["0", "1"])
+@pytest.mark.parametrize("d,hq,hkv,s", [(64, 8, 2, 777), (128, 4, 4, 300), (256, 4, 1, 130)])
+def test_prefill_batch_equals_single_prompts(monkeypatch, d, hq, hkv, s, paired):
+    """The sequences of a batch (their query blocks interleaved, heaviest first) against each
+    prompt alone under the same schedule: bit for bit."""
+    from powerinfer_x64_amd import runtime as rt
+    dev = device()
+    monkeypatch.setenv("PI_PREFILL_PAIRED", paired)
+    monkeypatch.setenv("PI_PREFILL_KSPLIT", "1")
+    rng = np.random.default_rng(d + s)
+    q, k, v = (to_dev(rng.standard_normal((3, s, h, d)).astype(np.float32), torch.float16) for h in (hq, hkv, hkv))
+    out = rt.attn_prefill(dev, q, k, v)
+    for i in range(3):
+        one = rt.attn_prefill(dev, q[i:i + 1].contiguous(), k[i:i + 1].contiguous(), v[i:i + 1].contiguous())
+        assert torch.equal(out[i], one[0])
