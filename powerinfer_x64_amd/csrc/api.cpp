@@ -658,6 +658,31 @@ int pi_attn_prefill(pi_handle h, const void* d_q, const void* d_k, const void* d
     return ws_end(h, s, "pi_attn_prefill");
 }
 
+// The f32 pool's prefill.  A key split's partials live in the handle's prefill workspace; a
+// launch under stream capture runs unsplit, so that a captured call neither allocates nor
+// shares a workspace with the calls beside its replays.
+static int prefill_f32(pi_handle h, const char* fn, const pi::KvGeom& g, const float* q, const int32_t* pt,
+                       int32_t max_pages, int32_t start, int32_t n_tok, int32_t n_q_heads, int32_t gqa_mode,
+                       float scale, float* out, hipStream_t s, const float* gate) {
+    const size_t need = pi::prefill_f32_ws_floats(start, n_tok, n_q_heads, g.n_kv_heads, g.head_dim);
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (need) PI_HIP(h, hipStreamIsCapturing(s, &cap), fn);
+    bool split = need && cap == hipStreamCaptureStatusNone;
+    int rc;
+    if (split) {
+        if ((rc = ws_begin(h, s, fn))) return rc;
+        // no memory for the partials: the launch runs unsplit
+        if (grow(h, &h->pfs_buf, &h->pfs_floats, need, s, fn, false)) {
+            (void)hipGetLastError();
+            split = false;
+        }
+    }
+    PI_HIP(h, pi::launch_prefill_f32(g, q, pt, max_pages, start, n_tok, n_q_heads, gqa_mode, scale, out,
+                                     split ? h->pfs_buf : nullptr, split ? h->pfs_floats : 0, s, gate),
+           fn);
+    return split ? ws_end(h, s, fn) : PI_OK;
+}
+
 int pi_attn_prefill_paged(pi_handle h, const void* d_q, pi_kv_pool pool,
                           const int32_t* d_page_table, int32_t max_pages, int32_t start_pos,
                           int32_t n_tok, int32_t n_q_heads, int32_t gqa_mode, float scale,
@@ -682,12 +707,9 @@ int pi_attn_prefill_paged(pi_handle h, const void* d_q, pi_kv_pool pool,
     if (n_tok == 0) return PI_OK;
     hipStream_t s = pick(h, stream);
     PI_HIP(h, hipSetDevice(h->device), "pi_attn_prefill_paged");
-    if (g.dtype == PI_F32) {  // straight from the pages, no workspace
-        PI_HIP(h, pi::launch_prefill_f32(g, static_cast<const float*>(d_q), d_page_table, max_pages,
-                                         start_pos, n_tok, n_q_heads, gqa_mode, scale, d_out, s),
-               "pi_attn_prefill_paged");
-        return PI_OK;
-    }
+    if (g.dtype == PI_F32)  // straight from the pages
+        return prefill_f32(h, "pi_attn_prefill_paged", g, static_cast<const float*>(d_q), d_page_table, max_pages,
+                           start_pos, n_tok, n_q_heads, gqa_mode, scale, d_out, s, nullptr);
     int rc;
     if ((rc = ws_begin(h, s, "pi_attn_prefill_paged"))) return rc;
     // straight from the f16 pages
@@ -1251,9 +1273,9 @@ static int attn_layer_step(pi_handle h, pi_attn_layer L, float* dq, float* dk, c
         if (dg && !dg_fused) PI_HIP(h, pi::launch_apply_gate(dout, dg, nq, s), "attention layer");
     } else if (n > 1 && L->kv_dtype == PI_F32) {
         // causal attention straight from the f32 pages, at f32 accuracy
-        PI_HIP(h, pi::launch_prefill_f32(L->pool->g, dq, L->d_pt, L->max_pages, prev, n, L->n_heads,
-                                         L->gqa_mode, scale, dout, s, dg_fused),
-               "attention layer");
+        if ((rc = prefill_f32(h, "attention layer", L->pool->g, dq, L->d_pt, L->max_pages, prev, n, L->n_heads,
+                              L->gqa_mode, scale, dout, s, dg_fused)))
+            return rc;
         if (dg && !dg_fused) PI_HIP(h, pi::launch_apply_gate(dout, dg, nq, s), "attention layer");
     } else {
         // one decode row per token over the paged cache: row i sees prev + i + 1 keys (the

@@ -1435,7 +1435,14 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_kernel(PrefillArgs a) {
     const int S = a.S, L = a.Sk, q_off = a.q_off;         // L: keys of the sequence after this chunk
     const int p0 = qb * WROWS + 32 * (rg % RG);           // this wave's first query row
     const int qpos = p0 + r;
-    const int n_tiles = (min(L, q_off + qb * WROWS + WROWS) + TK - 1) / TK;
+    // this workgroup's tiles [tb, n_tiles): the block's, or its piece of them under a key split
+    const int n_all = (min(L, q_off + qb * WROWS + WROWS) + BN - 1) / BN;  // in 64-key tiles
+    const int ksp = blockIdx.z, pieces = split_pieces(n_all, a.ksplit, a.kthr);
+    if (ksp >= pieces) return;  // uniform per workgroup
+    const int kper = (n_all + pieces - 1) / pieces;
+    const int tb = min(n_all, ksp * kper) * (BN / TK);
+    const int n_tiles = min(min(n_all, (ksp + 1) * kper) * (BN / TK),
+                            (min(L, q_off + qb * WROWS + WROWS) + TK - 1) / TK);
     const int w_keys = p0 < S ? min(L, q_off + p0 + 32) : 0;  // keys this wave's rows attend
 
     Tiles tl;
@@ -1446,9 +1453,9 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_kernel(PrefillArgs a) {
     tl.L = L;
     tl.n_pages = a.n_pages;
     tl.tid = tid;
-    tl.ids(0, tl.pid);
+    tl.ids(tb, tl.pid);
     tl.load();
-    tl.ids(1, tl.pid);
+    tl.ids(tb + 1, tl.pid);
 
     // Q^T operand: lane holds q[qpos][16 kk + 8 hh .. +7] as hi / lo
     bf16x8 qh[NKK], ql[NKK];
@@ -1542,11 +1549,11 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_kernel(PrefillArgs a) {
 
     auto stage = [&](int buf) { tl.stage(lds[buf], lds[buf] + NK, lds[buf] + 2 * NK, lds[buf] + 3 * NK); };
     stage(0);
-    if (1 < n_tiles) tl.load();
-    tl.ids(2, tl.pid);
+    if (tb + 1 < n_tiles) tl.load();
+    tl.ids(tb + 2, tl.pid);
     f32_barrier();
-    for (int t = 0; t < n_tiles; ++t) {
-        const int buf = t & 1;
+    for (int t = tb; t < n_tiles; ++t) {
+        const int buf = (t - tb) & 1;
         int nid[Tiles::NPG];
         tl.ids(t + 3, nid);
         auto next = [&]() {  // split tile t + 1, request tile t + 2
@@ -1582,10 +1589,17 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_kernel(PrefillArgs a) {
     const float m_o = xml[(ow * 2) * 64 + lane], l_o = xml[(ow * 2 + 1) * 64 + lane];
     const float M = fmaxf(m_run, m_o);
     const float w_s = fast_exp2(m_run - M), w_o = fast_exp2(m_o - M);
-    const float inv = 1.0f / (w_s * l_run + w_o * l_o);
+    const float l = w_s * l_run + w_o * l_o;
+    const bool split = pieces > 1;  // an unnormalised partial, for prefill_merge_kernel
+    const float inv = split ? 1.0f : 1.0f / l;
     const float f_s = w_s * inv, f_o = w_o * inv;
     const size_t row = (size_t)qpos * a.hq + head;
-    float* orow = a.out + row * D;
+    const size_t prow = (size_t)ksp * S * a.hq + row;
+    float* orow = split ? a.part_o + prow * D : a.out + row * D;
+    if (split && kh == 0 && hh == 0) {
+        a.part_ml[2 * prow] = M;
+        a.part_ml[2 * prow + 1] = l;
+    }
 #pragma unroll
     for (int i = 0; i < NDT; ++i)
         if ((i >= NDT / 2) == (kh == 1)) {
@@ -1597,7 +1611,7 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_kernel(PrefillArgs a) {
                 for (int e = 0; e < 4; ++e)
                     t[e] = o[i][4 * b + e] * f_s +
                            xch[((ow * (NDT / 2) + i % (NDT / 2)) * 16 + 4 * b + e) * 64 + lane] * f_o;
-                if (a.gate) {
+                if (a.gate && !split) {
                     const f32x4 gt = *reinterpret_cast<const f32x4*>(a.gate + row * D + d0);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) t[e] *= gate_sigmoid(gt[e]);
@@ -1636,7 +1650,14 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_256_kernel(PrefillArgs a) 
     const int S = a.S, L = a.Sk, q_off = a.q_off;         // L: keys of the sequence after this chunk
     const int p0 = qb * WROWS + 16 * (wave % RW);         // this wave's first query row
     const int qpos = p0 + c;
-    const int n_tiles = (min(L, q_off + qb * WROWS + WROWS) + TK - 1) / TK;
+    // this workgroup's tiles [tb, n_tiles): the block's, or its piece of them under a key split
+    const int n_all = (min(L, q_off + qb * WROWS + WROWS) + BN - 1) / BN;  // in 64-key tiles
+    const int ksp = blockIdx.z, pieces = split_pieces(n_all, a.ksplit, a.kthr);
+    if (ksp >= pieces) return;  // uniform per workgroup
+    const int kper = (n_all + pieces - 1) / pieces;
+    const int tb = min(n_all, ksp * kper) * (BN / TK);
+    const int n_tiles = min(min(n_all, (ksp + 1) * kper) * (BN / TK),
+                            (min(L, q_off + qb * WROWS + WROWS) + TK - 1) / TK);
     const int w_keys = p0 < S ? min(L, q_off + p0 + 16) : 0;  // keys this wave's rows attend
 
     Tiles tl;
@@ -1647,9 +1668,9 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_256_kernel(PrefillArgs a) 
     tl.L = L;
     tl.n_pages = a.n_pages;
     tl.tid = tid;
-    tl.ids(0, tl.pid);
+    tl.ids(tb, tl.pid);
     tl.load();
-    tl.ids(1, tl.pid);
+    tl.ids(tb + 1, tl.pid);
 
     // Q^T operand (B of K.Q^T): lane holds q[qpos][32 ks + 8 g .. +7] as hi / lo
     bf16x8 qh[NKS], ql[NKS];
@@ -1748,11 +1769,11 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_256_kernel(PrefillArgs a) 
 
     auto stage = [&](int buf) { tl.stage(lds[buf], lds[buf] + NK, lds[buf] + 2 * NK, lds[buf] + 3 * NK); };
     stage(0);
-    if (1 < n_tiles) tl.load();
-    tl.ids(2, tl.pid);
+    if (tb + 1 < n_tiles) tl.load();
+    tl.ids(tb + 2, tl.pid);
     f32_barrier();
-    for (int t = 0; t < n_tiles; ++t) {
-        const int buf = t & 1;
+    for (int t = tb; t < n_tiles; ++t) {
+        const int buf = (t - tb) & 1;
         int nid[Tiles::NPG];
         tl.ids(t + 3, nid);
         auto next = [&]() {  // split tile t + 1, request tile t + 2
@@ -1770,13 +1791,19 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_256_kernel(PrefillArgs a) 
     l_run += __shfl_xor(l_run, 16, 64);
     l_run += __shfl_xor(l_run, 32, 64);
     if (qpos >= S) return;
-    const float inv = 1.0f / l_run;
+    const bool split = pieces > 1;  // an unnormalised partial, for prefill_merge_kernel
+    const float inv = split ? 1.0f : 1.0f / l_run;
     const size_t row = (size_t)qpos * a.hq + head;
-    float* orow = a.out + row * D;
+    const size_t prow = (size_t)ksp * S * a.hq + row;
+    float* orow = split ? a.part_o + prow * D : a.out + row * D;
+    if (split && g == 0) {
+        a.part_ml[2 * prow] = m_run;
+        a.part_ml[2 * prow + 1] = l_run;
+    }
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
         f32x4 t = o[db] * inv;
-        if (a.gate) {
+        if (a.gate && !split) {
             const f32x4 gt = *reinterpret_cast<const f32x4*>(a.gate + row * D + 16 * db + 4 * g);
 #pragma unroll
             for (int e = 0; e < 4; ++e) t[e] *= gate_sigmoid(gt[e]);
@@ -2153,10 +2180,79 @@ hipError_t launch_prefill_pool(const KvGeom& g, const void* q, int32_t q_f32, co
     return launch_merge(D, a, 1, q0, wrows, out, s);
 }
 
+namespace {
+struct F32Sched {
+    int hpw, wrows, ksplit, kthr, q0;  // q0: first query row of a split block
+};
+
+// The f32 prefill's key split.  One workgroup (a block of wrows rows) runs on a CU at a time,
+// about 3 us a 64-key tile, so a launch with fewer blocks than CUs takes its longest block's
+// tiles.  Its blocks then run in up to four pieces of at most kthr tiles, the smallest for
+// which all pieces fit the CUs once, if that shortens the longest by the 4 tiles that pay for
+// the merge launch: 64 tokens over 4096, 32/32 heads, D 128 190 -> 64 us, 1024 over 8192 at
+// 16/2 heads D 256 762 -> 463, a fresh 1000-token layer prompt there 107 -> 70.  A launch that
+// fills the CUs runs whole: pieces of the average CU's tiles ran 1000 tokens at 32/32 heads,
+// D 128 in 87.6 us against 84.5.  PI_PREFILL_KSPLIT=n forces the pieces of the longest block
+// (1: none).
+F32Sched f32_sched(int q_off, int n_tok, int n_q_heads, int n_kv_heads) {
+    F32Sched sc;
+    const bool multiple = n_q_heads % n_kv_heads == 0;
+    const int group = (n_q_heads + n_kv_heads - 1) / n_kv_heads;
+    sc.hpw = !multiple ? 1 : group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1);
+    sc.wrows = 128 / sc.hpw;
+    sc.ksplit = 1;
+    sc.kthr = 0;
+    sc.q0 = n_tok;
+    const long long hsets = (long long)n_kv_heads * (group / sc.hpw), n_cu = cu_count();
+    const int nqb = (n_tok + sc.wrows - 1) / sc.wrows;
+    auto tiles = [&](int qb) {
+        return (int)((std::min<long long>((long long)q_off + n_tok, (long long)q_off + (qb + 1LL) * sc.wrows) + BN - 1) / BN);
+    };
+    const int most = tiles(nqb - 1);
+    int p = most;
+    if (const char* env = std::getenv("PI_PREFILL_KSPLIT")) {
+        const int k = std::max(1, std::min(4, std::atoi(env)));
+        p = (most + k - 1) / k;
+    } else {
+        if (n_cu <= 0 || most < 5 || nqb * hsets >= n_cu) return sc;
+        auto fits = [&](int q) {
+            long long n = 0;
+            for (int qb = 0; qb < nqb; ++qb) n += (tiles(qb) + q - 1) / q;
+            return n * hsets <= n_cu;
+        };
+        if (!fits(most - 1)) return sc;
+        int lo = (most + 3) / 4, hi = most - 1;  // fits is monotone
+        while (lo < hi) {
+            const int mid = (lo + hi) / 2;
+            if (fits(mid)) hi = mid;
+            else lo = mid + 1;
+        }
+        p = lo;
+        if (most < p + 4) return sc;
+    }
+    if (p >= most) return sc;
+    sc.kthr = p;
+    sc.ksplit = (most + p - 1) / p;
+    for (int qb = 0; qb < nqb; ++qb)
+        if (tiles(qb) > p) {
+            sc.q0 = qb * sc.wrows;
+            break;
+        }
+    return sc;
+}
+}  // namespace
+
+size_t prefill_f32_ws_floats(int32_t q_off, int32_t n_tok, int32_t n_q_heads, int32_t n_kv_heads,
+                             int32_t head_dim) {
+    if (q_off < 0 || n_tok <= 0 || n_q_heads <= 0 || n_kv_heads <= 0) return 0;
+    const F32Sched sc = f32_sched(q_off, n_tok, n_q_heads, n_kv_heads);
+    return sc.ksplit > 1 ? (size_t)sc.ksplit * n_tok * n_q_heads * (head_dim + 2) : 0;
+}
+
 hipError_t launch_prefill_f32(const KvGeom& g, const float* q, const int32_t* page_table,
                               int32_t max_pages, int32_t q_off, int32_t n_tok, int32_t n_q_heads,
-                              int32_t gqa_mode, float scale, float* out, hipStream_t s,
-                              const float* gate) {
+                              int32_t gqa_mode, float scale, float* out, float* ws, size_t ws_floats,
+                              hipStream_t s, const float* gate) {
     const int D = g.head_dim;
     if (g.dtype != 0 || (D != 64 && D != 128 && D != 256) || q_off < 0 || n_tok < 1 || max_pages < 1)
         return hipErrorInvalidValue;
@@ -2185,9 +2281,17 @@ hipError_t launch_prefill_f32(const KvGeom& g, const float* q, const int32_t* pa
     a.vstride = g.vstride;
     a.n_pages = g.n_pages;
     a.ksplit = 1;
-    const int hpw = !multiple ? 1 : a.group % 4 == 0 ? 4 : (a.group % 2 == 0 ? 2 : 1);
-    const int wrows = 128 / hpw;
-    const dim3 grid((unsigned)(g.n_kv_heads * (a.group / hpw)), (unsigned)((n_tok + wrows - 1) / wrows));
+    F32Sched sc = f32_sched(q_off, n_tok, n_q_heads, g.n_kv_heads);
+    const int hpw = sc.hpw;
+    const size_t rows = (size_t)n_tok * n_q_heads;
+    if (sc.ksplit > 1 && ws && ws_floats >= (size_t)sc.ksplit * rows * (D + 2)) {
+        a.ksplit = sc.ksplit;
+        a.kthr = sc.kthr;
+        a.part_o = ws;
+        a.part_ml = ws + (size_t)sc.ksplit * rows * D;
+    }
+    const dim3 grid((unsigned)(g.n_kv_heads * (a.group / hpw)), (unsigned)((n_tok + sc.wrows - 1) / sc.wrows),
+                    (unsigned)a.ksplit);
 #define PI_F32(DD)                                                                                \
     switch (hpw) {                                                                                \
         case 4: hipLaunchKernelGGL((prefill_f32_kernel<DD, 4>), grid, dim3(512), 0, s, a); break; \
@@ -2203,7 +2307,9 @@ hipError_t launch_prefill_f32(const KvGeom& g, const float* q, const int32_t* pa
     } else if (D == 128) PI_F32(128)
     else PI_F32(64)
 #undef PI_F32
-    return hipGetLastError();
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || a.ksplit == 1) return e;
+    return launch_merge(D, a, 1, sc.q0, sc.wrows, out, s);
 }
 
 }  // namespace pi

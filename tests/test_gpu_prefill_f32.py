@@ -69,3 +69,54 @@ def test_f32_prefill_page_outside_the_pool(d):
         v[16 * p:16 * p + 16] = 0
     out = rt.attn_prefill_paged(dev, to_dev(q), c.pool, to_dev(row), c.prev).cpu().numpy()
     _check(c, out, [0, 20, 39], k, v)
+
+
+@pytest.mark.parametrize("ksplit", ["2", "3", "4"])
+@pytest.mark.parametrize("prev,n,hq,hkv,d", [(0, 300, 4, 1, 64), (500, 130, 3, 3, 128), (1000, 33, 5, 2, 128),
+                                             (64, 257, 8, 4, 256), (2000, 16, 16, 2, 256)])
+def test_f32_prefill_key_splits(monkeypatch, prev, n, hq, hkv, d, ksplit):
+    """Forced key splits: pieces of the longest blocks, short blocks whole, pieces that hold no key
+    of a row, through the layer's gated step as well as the paged entry."""
+    from powerinfer_x64_amd import runtime as rt
+    dev = device()
+    c = Chunk(np.random.default_rng(prev + n + d), prev, n, hq, hkv, d)
+    monkeypatch.setenv("PI_PREFILL_KSPLIT", ksplit)
+    out = c.gpu(dev, pool_dtype=torch.float32)
+    _check(c, out, sorted({0, 1, 31, n // 2, n - 1} & set(range(n))))
+    if prev == 0:
+        g = np.random.default_rng(1).standard_normal((n, hq, d)).astype(np.float32)
+        got = []
+        for k in (ksplit, "1"):
+            monkeypatch.setenv("PI_PREFILL_KSPLIT", k)
+            layer = rt.AttnLayer(dev, n, hq, hkv, d, torch.float32, rope_base=c.theta)
+            got.append(layer.forward_dev(*(to_dev(x) for x in (c.q, c.k, c.v, g))))
+        assert float((got[0] - got[1]).abs().max()) <= 2.0 ** -18 * float(np.abs(c.v).max())
+
+
+def test_f32_prefill_automatic_split_and_capture():
+    """Few queries over a long history: the launch splits by itself, and not under capture; the
+    replays equal the eager unsplit call bit for bit."""
+    import os
+    from powerinfer_x64_amd import runtime as rt
+    dev = device()
+    c = Chunk(np.random.default_rng(7), 3000, 20, 8, 2, 128)
+    out = c.gpu(dev, pool_dtype=torch.float32)
+    _check(c, out, [0, 7, 19])
+    q = to_dev(c.prepared(f32=True)[0])
+    os.environ["PI_PREFILL_KSPLIT"] = "1"
+    try:
+        ref = rt.attn_prefill_paged(dev, q, c.pool, c.row_dev, c.prev)
+    finally:
+        del os.environ["PI_PREFILL_KSPLIT"]
+    o = torch.zeros_like(ref)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        rt.attn_prefill_paged(dev, q, c.pool, c.row_dev, c.prev, out=o)
+    for _ in range(3):
+        o.zero_()
+        rt.attn_prefill_paged(dev, q, c.pool, c.row_dev, c.prev)  # eager work between replays
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o, ref)
