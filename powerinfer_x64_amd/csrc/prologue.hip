@@ -531,7 +531,7 @@ __device__ __forceinline__ void prologue_page(float* __restrict__ k, const float
     }
 }
 
-template <typename PT, int EPL>
+template <typename PT, int EPL, bool BYPAGE>
 __global__ __launch_bounds__(256) void attn_prologue_vec_kernel(
     float* __restrict__ q, float* __restrict__ k, const float* __restrict__ v,
     const float* __restrict__ qn, const float* __restrict__ kn, float eps, RopeFreqs f,
@@ -540,18 +540,21 @@ __global__ __launch_bounds__(256) void attn_prologue_vec_kernel(
     constexpr int D = 64 * EPL;
     __shared__ float cs_s[2][128];  // cos, sin of pair i at this token's position
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    // ppn > 0: the first n_seq * ppn * n_kv_heads workgroups take the K / V side by page
+    // BYPAGE: the first n_seq * ppn * n_kv_heads workgroups take the K / V side by page
     // (dispatched first, so they run beside the token workgroups), and the token workgroups
-    // after them only the q heads
+    // after them only the q heads.  A kernel of its own, without the V rows' registers (76
+    // instead of 114 at EPL 4), so that the rows can be requested before the cos / sin table
+    // without costing residents: 1024 tokens, 16/2 heads, D 256 12.8 -> 10.3 us; 4096, 32/8,
+    // D 128 46.4 -> 40.6.
     const int toks = n_seq * n_tok;
-    const int n_pg = ppn > 0 ? n_seq * ppn * g.n_kv_heads : 0;
-    if ((int)blockIdx.x < n_pg) {
+    const int n_pg = BYPAGE ? n_seq * ppn * g.n_kv_heads : 0;
+    if (BYPAGE && (int)blockIdx.x < n_pg) {
         if (blockIdx.y == 0)  // launches that split the token's heads over y: one copy
             prologue_page<PT, EPL>(k, v, kn, eps, f, n_pairs, neox, g, pt, max_pages, start_pos,
                                    n_tok, norm_d, (int)blockIdx.x, ppn);
         return;
     }
-    const int hkv = g.n_kv_heads, heads = ppn > 0 ? hq : hq + hkv;
+    const int hkv = g.n_kv_heads, heads = BYPAGE ? hq : hq + hkv;
     const bool table = gridDim.y == 1;  // uniform per launch: the token remap below
     // A prompt launch keeps each run of 16 consecutive tokens (a page of K and V when
     // the prompt starts on a page) on one XCD: workgroups are dispatched round-robin
@@ -566,6 +569,39 @@ __global__ __launch_bounds__(256) void attn_prologue_vec_kernel(
     const int t = u % n_tok, sq = u / n_tok;
     const int pos = start_pos.of(sq) + t;
     start_pos.write_ctx();
+    const int e0 = EPL * lane;  // this lane's first element of a row
+    const int per = (heads + gridDim.y - 1) / gridDim.y;
+    const int h1 = min(heads, (int)(blockIdx.y + 1) * per);
+    auto row_of = [&](int head) {
+        return BYPAGE || head < hq ? q + (((size_t)sq * n_tok + t) * hq + head) * D
+                                   : k + (((size_t)sq * n_tok + t) * hkv + (head - hq)) * D;
+    };
+    // A wavefront's heads are head0, head0 + 4, ...: the rows of up to MH of them (and the V
+    // rows of its K heads) are loaded before any is processed, so their loads overlap.
+    constexpr int MH = 6;
+    float xs[MH][EPL], vs[MH][EPL];
+    auto load_rows = [&](int head0) {
+#pragma unroll
+        for (int m = 0; m < MH; ++m) {
+            const int head = head0 + 4 * m;
+            if (head < h1) {
+                load_vec<EPL>(xs[m], row_of(head) + e0);
+                if (!BYPAGE && head >= hq)
+                    load_vec<EPL>(vs[m], v + (((size_t)sq * n_tok + t) * hkv + (head - hq)) * D + e0);
+            }
+        }
+    };
+    // the norm weights (the same for every row of a kind) are read once, beside the rows
+    float qw[EPL], kw[EPL];
+    auto load_weights = [&]() {
+        if (qn) load_vec<EPL>(qw, qn + e0);
+        if (!BYPAGE && kn) load_vec<EPL>(kw, kn + e0);
+    };
+    const int hfirst = blockIdx.y * per + wv;
+    if (BYPAGE) {
+        load_rows(hfirst);
+        load_weights();
+    }
     // cos / sin of the workgroup's token position, once per pair (every thread of the
     // workgroup works on that token)
     for (int i = threadIdx.x; i < n_pairs; i += 256) {
@@ -578,39 +614,14 @@ __global__ __launch_bounds__(256) void attn_prologue_vec_kernel(
         *c = cs_s[0][i];
         *sn = cs_s[1][i];
     };
-    const int e0 = EPL * lane;  // this lane's first element of a row
-    const int per = (heads + gridDim.y - 1) / gridDim.y;
-    const int h1 = min(heads, (int)(blockIdx.y + 1) * per);
-    auto row_of = [&](int head) {
-        return head < hq ? q + (((size_t)sq * n_tok + t) * hq + head) * D
-                         : k + (((size_t)sq * n_tok + t) * hkv + (head - hq)) * D;
-    };
-    // A wavefront's heads are head0, head0 + 4, ...: the rows of up to MH of them (and the V
-    // rows of its K heads) are loaded before any is processed, so their loads overlap.
-    constexpr int MH = 6;
-    // the norm weights (the same for every row of a kind) are read once, beside the rows
-    float qw[EPL], kw[EPL];
-    bool wl = false;
-    for (int head0 = blockIdx.y * per + wv; head0 < h1; head0 += 4 * MH) {
-        float xs[MH][EPL], vs[MH][EPL];
-#pragma unroll
-        for (int m = 0; m < MH; ++m) {
-            const int head = head0 + 4 * m;
-            if (head < h1) {
-                load_vec<EPL>(xs[m], row_of(head) + e0);
-                if (head >= hq) load_vec<EPL>(vs[m], v + (((size_t)sq * n_tok + t) * hkv + (head - hq)) * D + e0);
-            }
-        }
-        if (!wl) {
-            if (qn) load_vec<EPL>(qw, qn + e0);
-            if (kn) load_vec<EPL>(kw, kn + e0);
-            wl = true;
-        }
+    for (int head0 = hfirst; head0 < h1; head0 += 4 * MH) {
+        if (!BYPAGE || head0 != hfirst) load_rows(head0);
+        if (!BYPAGE && head0 == hfirst) load_weights();
 #pragma unroll
         for (int m = 0; m < MH; ++m) {
             const int head = head0 + 4 * m;
             if (head >= h1) break;
-            const bool is_q = head < hq;
+            const bool is_q = BYPAGE || head < hq;
             const int kvh = head - hq;
             float* x = row_of(head);
             float* xv = xs[m];
@@ -752,7 +763,8 @@ hipError_t launch_attn_prologue(float* q, float* k, const float* v, const float*
                                          (size_t)2 * kPageTokens * n_pairs * sizeof(float)
                                    : 0;
 #define PI_PROLOGUE_VEC(PT, E)                                                                       \
-    hipLaunchKernelGGL((attn_prologue_vec_kernel<PT, E>), grid_v, dim3(256), lds, s, q, k, v,       \
+    hipLaunchKernelGGL((by_page ? attn_prologue_vec_kernel<PT, E, true>                              \
+                                : attn_prologue_vec_kernel<PT, E, false>), grid_v, dim3(256), lds, s, q, k, v,       \
                        q_norm_w, k_norm_w, eps, freqs, n_pairs, neox, g, page_table, max_pages, spv, \
                        n_seq, n_tok, n_q_heads, norm_d, ppn)
         const bool hp = g.dtype == 1;
