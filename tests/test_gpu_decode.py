@@ -227,3 +227,27 @@ def test_one_sequence_short_contexts(pool_dtype, d, hq, hkv, length):
         assert err <= 2e-3, f"max-abs {err}"
     else:
         _check_f16(case, got)
+
+
+def test_workspace_ordered_across_streams():
+    """Calls on two streams in turn share the handle's partials; the event between them orders the
+    device's streams, so every result is the one of a call alone, bit for bit."""
+    from powerinfer_x64_amd import runtime as rt
+    dev = device()
+    rng = np.random.default_rng(0x57E)
+    case = PagedCase(rng, [3000, 1700], 16, 4, 128)
+    case.gpu_build(dev, torch.float16)
+    ctx = to_dev(np.array(case.lens, np.int32))
+    qs = [to_dev(rng.standard_normal((2, 16, 128)).astype(np.float32)) for _ in range(2)]
+    ref = [rt.attn_decode(dev, q, case.pool, case.pt, ctx) for q in qs]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    outs = [[torch.empty_like(q) for _ in range(16)] for q in qs]
+    torch.cuda.synchronize()
+    for i in range(16):
+        for s, q, o in zip(streams, qs, outs):
+            with torch.cuda.stream(s):
+                rt.attn_decode(dev, q, case.pool, case.pt, ctx, out=o[i])
+    torch.cuda.synchronize()
+    for r, o in zip(ref, outs):
+        assert all(torch.equal(r, x) for x in o)
