@@ -598,10 +598,8 @@ __global__ __launch_bounds__(256) void attn_prologue_vec_kernel(
         if (!BYPAGE && kn) load_vec<EPL>(kw, kn + e0);
     };
     const int hfirst = blockIdx.y * per + wv;
-    if (BYPAGE) {
-        load_rows(hfirst);
-        load_weights();
-    }
+    load_rows(hfirst);
+    load_weights();
     // cos / sin of the workgroup's token position, once per pair (every thread of the
     // workgroup works on that token)
     for (int i = threadIdx.x; i < n_pairs; i += 256) {
@@ -615,8 +613,7 @@ __global__ __launch_bounds__(256) void attn_prologue_vec_kernel(
         *sn = cs_s[1][i];
     };
     for (int head0 = hfirst; head0 < h1; head0 += 4 * MH) {
-        if (!BYPAGE || head0 != hfirst) load_rows(head0);
-        if (!BYPAGE && head0 == hfirst) load_weights();
+        if (head0 != hfirst) load_rows(head0);
 #pragma unroll
         for (int m = 0; m < MH; ++m) {
             const int head = head0 + 4 * m;
