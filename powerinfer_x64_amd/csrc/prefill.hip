@@ -101,6 +101,10 @@ struct PrefillArgs {
 
 __device__ __forceinline__ float gate_sigmoid(float g) { return 1.0f / (1.0f + expf(-g)); }
 
+// A row's normalisation, 1 / its softmax sum.  A row whose every key is on a page outside the
+// pool has the sum 0 and gets zeros, as in the decode.
+__device__ __forceinline__ float inv_sum(float l) { return l == 0.f ? 0.f : 1.0f / l; }
+
 // Pieces of a query block of n key tiles under a key split (1: the block runs whole).
 __host__ __device__ __forceinline__ int split_pieces(int n, int ksplit, int kthr) {
     return ksplit > 1 && kthr > 0 && n > kthr ? min(ksplit, (n + kthr - 1) / kthr) : 1;
@@ -1332,7 +1336,10 @@ struct F32Tiles {
     int L, n_pages, tid;
     int pid[NPG];
     f32x4 pre[NF];
-    unsigned bad;  // pages of the loaded tile that are outside the pool: they hold no tokens (zeros)
+    // pages of the loaded tile that are outside the pool.  They hold no tokens: page 0 is loaded in
+    // their place and split as zeros (a weight of 0 times its values must not give NaN), and
+    // compute() masks their keys by the bits that stage() returns with the tile.
+    unsigned bad;
 
     __device__ __forceinline__ void ids(int t, int (&id)[NPG]) const {
 #pragma unroll
@@ -1354,7 +1361,7 @@ struct F32Tiles {
                 page + (i >= 0 ? voff + 16 * (size_t)((i & ~63) + 4 * (i & 15) + ((i >> 4) & 3)) : 16 * (size_t)w));
         }
     }
-    __device__ __forceinline__ void stage(bf16x8* kh, bf16x8* kl, bf16x8* vh, bf16x8* vl) {
+    __device__ __forceinline__ unsigned stage(bf16x8* kh, bf16x8* kl, bf16x8* vh, bf16x8* vl) {
         if (bad) {  // here and not at the load, whose result a select would wait for
 #pragma unroll
             for (int j = 0; j < NF; ++j)
@@ -1384,6 +1391,7 @@ struct F32Tiles {
                 reinterpret_cast<bf16x4*>(vl)[at] = l;
             }
         }
+        return bad;
     }
 };
 
@@ -1478,7 +1486,8 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_kernel(PrefillArgs a) {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, acc, 0, 0, 0);
     };
     const float cs = a.qk_scale;
-    auto compute = [&](int k0, int buf) {  // keys k0 .. k0 + 31, rows 32 kh .. of the tile
+    // keys k0 .. k0 + 31, rows 32 kh .. of the tile; off: its 16-key pages outside the pool
+    auto compute = [&](int k0, int buf, unsigned off) {
         f32x16 st = {};
 #pragma unroll
         for (int kk = 0; kk < NKK; ++kk) {
@@ -1502,6 +1511,11 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_kernel(PrefillArgs a) {
                 const int key = k0 + 8 * (i >> 2) + 4 * hh + (i & 3);
                 if (key >= L || key > q_off + qpos) st[i] = -INFINITY;
             }
+        }
+        if (off) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                if (off >> (i >> 3) & 1) st[i] = -INFINITY;
         }
         float mx = st[0];
 #pragma unroll
@@ -1547,8 +1561,8 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_kernel(PrefillArgs a) {
         }
     };
 
-    auto stage = [&](int buf) { tl.stage(lds[buf], lds[buf] + NK, lds[buf] + 2 * NK, lds[buf] + 3 * NK); };
-    stage(0);
+    auto stage = [&](int buf) { return tl.stage(lds[buf], lds[buf] + NK, lds[buf] + 2 * NK, lds[buf] + 3 * NK); };
+    unsigned off = stage(0), off_next = 0;  // the computed tile's and the next one's bad pages
     if (tb + 1 < n_tiles) tl.load();
     tl.ids(tb + 2, tl.pid);
     f32_barrier();
@@ -1557,15 +1571,16 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_kernel(PrefillArgs a) {
         int nid[Tiles::NPG];
         tl.ids(t + 3, nid);
         auto next = [&]() {  // split tile t + 1, request tile t + 2
-            if (t + 1 < n_tiles) stage(buf ^ 1);
+            if (t + 1 < n_tiles) off_next = stage(buf ^ 1);
             if (t + 2 < n_tiles) tl.load();
 #pragma unroll
             for (int p = 0; p < Tiles::NPG; ++p) tl.pid[p] = nid[p];
         };
         const int k0 = t * TK + 32 * kh;
         if (kh == 0) next();
-        if (k0 < w_keys) compute(k0, buf);
+        if (k0 < w_keys) compute(k0, buf, off >> (2 * kh) & 3);
         if (kh == 1) next();
+        off = off_next;
         f32_barrier();
     }
 
@@ -1591,7 +1606,7 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_kernel(PrefillArgs a) {
     const float w_s = fast_exp2(m_run - M), w_o = fast_exp2(m_o - M);
     const float l = w_s * l_run + w_o * l_o;
     const bool split = pieces > 1;  // an unnormalised partial, for prefill_merge_kernel
-    const float inv = split ? 1.0f : 1.0f / l;
+    const float inv = split ? 1.0f : inv_sum(l);
     const float f_s = w_s * inv, f_o = w_o * inv;
     const size_t row = (size_t)qpos * a.hq + head;
     const size_t prow = (size_t)ksp * S * a.hq + row;
@@ -1693,7 +1708,8 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_256_kernel(PrefillArgs a) 
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, acc, 0, 0, 0);
     };
     const float cs = a.qk_scale;
-    auto compute = [&](int k0, int buf) {  // S^T for keys k0 + 16 kb + 4 g + r
+    // S^T for keys k0 + 16 kb + 4 g + r; off: the tile's 16-key pages outside the pool
+    auto compute = [&](int k0, int buf, unsigned off) {
         f32x4 st[NKB];
 #pragma unroll
         for (int kb = 0; kb < NKB; ++kb) st[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1721,6 +1737,11 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_256_kernel(PrefillArgs a) 
                     const int key = k0 + 16 * kb + 4 * g + r;
                     if (key >= L || key > q_off + qpos) st[kb][r] = -INFINITY;
                 }
+        }
+        if (off) {
+#pragma unroll
+            for (int kb = 0; kb < NKB; ++kb)
+                if (off >> kb & 1) st[kb] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
         }
         float mx = st[0][0];
 #pragma unroll
@@ -1767,8 +1788,8 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_256_kernel(PrefillArgs a) 
         }
     };
 
-    auto stage = [&](int buf) { tl.stage(lds[buf], lds[buf] + NK, lds[buf] + 2 * NK, lds[buf] + 3 * NK); };
-    stage(0);
+    auto stage = [&](int buf) { return tl.stage(lds[buf], lds[buf] + NK, lds[buf] + 2 * NK, lds[buf] + 3 * NK); };
+    unsigned off = stage(0), off_next = 0;  // the computed tile's and the next one's bad pages
     if (tb + 1 < n_tiles) tl.load();
     tl.ids(tb + 2, tl.pid);
     f32_barrier();
@@ -1777,14 +1798,15 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_256_kernel(PrefillArgs a) 
         int nid[Tiles::NPG];
         tl.ids(t + 3, nid);
         auto next = [&]() {  // split tile t + 1, request tile t + 2
-            if (t + 1 < n_tiles) stage(buf ^ 1);
+            if (t + 1 < n_tiles) off_next = stage(buf ^ 1);
             if (t + 2 < n_tiles) tl.load();
 #pragma unroll
             for (int p = 0; p < Tiles::NPG; ++p) tl.pid[p] = nid[p];
         };
         if (wave < 4) next();
-        if (t * TK < w_keys) compute(t * TK, buf);
+        if (t * TK < w_keys) compute(t * TK, buf, off);
         if (wave >= 4) next();
+        off = off_next;
         f32_barrier();
     }
 
@@ -1792,7 +1814,7 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_256_kernel(PrefillArgs a) 
     l_run += __shfl_xor(l_run, 32, 64);
     if (qpos >= S) return;
     const bool split = pieces > 1;  // an unnormalised partial, for prefill_merge_kernel
-    const float inv = split ? 1.0f : 1.0f / l_run;
+    const float inv = split ? 1.0f : inv_sum(l_run);
     const size_t row = (size_t)qpos * a.hq + head;
     const size_t prow = (size_t)ksp * S * a.hq + row;
     float* orow = split ? a.part_o + prow * D : a.out + row * D;
@@ -1866,7 +1888,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const float* __restr
             L += w * ml[m][k][1];
             acc += w * o[m][k];
         }
-        acc *= 1.0f / L;
+        acc *= inv_sum(L);
         if (gate) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[e] *= gate_sigmoid(gt[m][e]);

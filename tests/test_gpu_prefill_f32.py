@@ -53,22 +53,37 @@ def test_f32_prefill_max_rises_late(d):
     _check(c, out, [0, 31, 63, 64, 130, 199])
 
 
+# history, chunk and the pages made invalid: inside and at the edges of the 32-key halves and the
+# 32 / 64-key tiles, whole tiles (first, last), the chunk's own pages, and every page of a row
+@pytest.mark.parametrize("ksplit", ["1", "3"])
 @pytest.mark.parametrize("d", [64, 128, 256])
-def test_f32_prefill_page_outside_the_pool(d):
-    """A page id outside the pool reads as zero keys and values."""
+@pytest.mark.parametrize("prev,n,bad", [(150, 40, (3, 9)), (150, 40, (4, 5, 6, 7, 11)), (0, 100, (0, 1)),
+                                        (200, 70, (0, 1, 2, 3, 12, 13, 16)), (37, 60, tuple(range(6)))])
+def test_f32_prefill_pages_outside_the_pool_hold_no_tokens(monkeypatch, prev, n, bad, d, ksplit):
+    """Page-table entries outside [0, n_pages) hold no tokens, as for the decode and the f16
+    prefill: their keys are left out of the softmax, and a row with no other key gets zeros."""
     from powerinfer_x64_amd import runtime as rt
     dev = device()
-    c = Chunk(np.random.default_rng(d + 1), 150, 40, 4, 2, d)
+    monkeypatch.setenv("PI_PREFILL_KSPLIT", ksplit)
+    c = Chunk(np.random.default_rng(d + prev), prev, n, 4, 2, d)
     c.gpu(dev, pool_dtype=torch.float32)
     q, k, v = c.prepared(f32=True)
-    row = c.row.copy()
-    row[3], row[9] = c.n_pages, -1
-    k, v = k.copy(), v.copy()
-    for p in (3, 9):
-        k[16 * p:16 * p + 16] = 0
-        v[16 * p:16 * p + 16] = 0
-    out = rt.attn_prefill_paged(dev, to_dev(q), c.pool, to_dev(row), c.prev).cpu().numpy()
-    _check(c, out, [0, 20, 39], k, v)
+    row, keep = c.row.copy(), np.ones(prev + n, bool)
+    for i, p in enumerate(bad):
+        row[p] = (-1, c.n_pages, c.n_pages + 3, -7)[i % 4]
+        keep[16 * p:16 * p + 16] = False
+    out = rt.attn_prefill_paged(dev, to_dev(q), c.pool, to_dev(row), prev).cpu().numpy()
+    dec = rt.attn_decode(dev, to_dev(q), c.pool, to_dev(np.tile(row, (n, 1))),
+                         to_dev(np.arange(prev + 1, prev + n + 1, dtype=np.int32))).cpu().numpy()
+    for i in range(n):
+        m = keep[:prev + i + 1]
+        kk, vv = k[:prev + i + 1][m], v[:prev + i + 1][m]
+        if not m.any():
+            assert not out[i].any() and not dec[i].any(), f"row {i} has no keys"
+            continue
+        ref, tol = orc.attn_decode(q[i], kk, vv), _bound(q[i:i + 1], kk, v)
+        assert float(np.abs(out[i] - ref).max()) <= tol, f"row {i}"
+        assert float(np.abs(out[i] - dec[i]).max()) <= 2 * tol, f"row {i} against the decode"
 
 
 @pytest.mark.parametrize("ksplit", ["2", "3", "4"])
