@@ -736,7 +736,7 @@ __global__ __launch_bounds__(64 * PrefillCfg<D>::NW, 1) void prefill_fa_kernel(P
             }
         }
     } else if (qpos < S) {
-        const float inv = 1.0f / l_run;
+        const float inv = inv_sum(l_run);
         const size_t ro = (((size_t)b * S + qpos) * a.hq + head) * D;
         float* orow = a.out + ro;
 #pragma unroll
@@ -1257,7 +1257,7 @@ __global__ __launch_bounds__(512, 1) void prefill_fa256_kernel(PrefillArgs a) {
             }
         }
     } else if (qpos < S) {
-        const float inv = 1.0f / l_run;
+        const float inv = inv_sum(l_run);
         const size_t ro = (((size_t)b * S + qpos) * a.hq + head) * D;
         float* orow = a.out + ro;
 #pragma unroll

@@ -256,6 +256,27 @@ def test_paged_prefill_page_ids_outside_the_pool_hold_no_tokens(d):
     _check(out, np.stack(parallel_map(ref_row, range(c.n))), "pages outside the pool")
 
 
+@pytest.mark.parametrize("ksplit", ["1", "2", "4"])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_paged_prefill_rows_without_keys_are_zero(monkeypatch, d, ksplit):
+    """Every page of the first rows outside the pool: those rows have no key and get zeros, as
+    from the decode, whether the launch splits its keys or not; the other rows see theirs."""
+    from powerinfer_x64_amd import runtime as rt
+    dev = device()
+    monkeypatch.setenv("PI_PREFILL_KSPLIT", ksplit)
+    c = Chunk(np.random.default_rng(0xE0 + d), 40, 300, 8, 2, d)
+    c.gpu(dev)
+    row = c.row.copy()
+    row[:10] = -1  # keys 0 .. 159: rows 0 .. 119 have none
+    out = rt.attn_prefill_paged(dev, c.q16, c.pool, to_dev(row), c.prev).cpu().numpy()
+    dec = rt.attn_decode(dev, c.q16[:2].float(), c.pool, to_dev(np.tile(row, (2, 1))),
+                         to_dev(np.array([41, 42], np.int32))).cpu().numpy()
+    assert not out[:120].any() and not dec.any()
+    q, k, v = c.prepared()
+    ref = np.stack(parallel_map(lambda i: orc.attn_decode(q[i], k[160:41 + i], v[160:41 + i]), range(120, 300)))
+    _check(out[120:], ref, "rows with keys")
+
+
 @pytest.mark.parametrize("paired,ksplit", [("1", None), (None, "2"), (None, "3"), (None, "4")])
 @pytest.mark.parametrize("prev,n,hq,hkv,d", [(700, 150, 32, 8, 128), (1000, 129, 16, 2, 256),
                                              (300, 129, 16, 4, 64)])
