@@ -18,6 +18,7 @@
 // projection >= 0.
 #include "pi_device.hpp"
 #include "pi_launch.hpp"
+#include "tq_sched.hpp"
 
 namespace pi {
 namespace {
@@ -712,37 +713,38 @@ hipError_t launch_tq_append(const TqPool& t, const float* k, const float* v,
     if ((items + 3) / 4 > 0x7fffffffLL) return hipErrorInvalidValue;
     const dim3 grid((unsigned)((items + 3) / 4));
     if (t.g.head_dim == 128 || t.g.head_dim == 256) {
-        // Rows a group (r): as many as leave the chip enough wavefronts.  A group's coordinates
-        // are split over D / 64 wavefronts, until the launch is so large that reading the rows'
-        // LDS values in each of them costs more than the shorter chains save.  Measured, D 128
-        // (8 heads): 8 rows 8.2 us (r 1), 2048 rows 13.8 (r 2; 16.2 at r 1), 8192 28.4 (r 4; 32.8
-        // at r 2), 16 384 44.5 (r 8; 46.5 at r 4), 131 072 212 (one wavefront a group; 231 split);
-        // D 256 (2 heads): 2 rows 12.6 (23.6 unsplit), 2048 33.9 (r 4), 32 768 236.
-        const long long units = items * (t.g.head_dim / 128);
-        const int r = units >= 8192 ? 8 : units >= 4096 ? 4 : units >= 2048 ? 2 : 1;
-        const int wpr = units >= 65536 ? 1 : t.g.head_dim / 64;
-        // groups of r aligned positions that n_tok positions from anywhere can touch
-        const long long n_grp = ((long long)n_tok + r - 2) / r + 1;
-        const long long waves = n_grp * n_seq * t.g.n_kv_heads * wpr;
-        if ((waves + 3) / 4 > 0x7fffffffLL || n_grp > 0x7fffffffLL) return hipErrorInvalidValue;
+        const sched::TqAppendPlan p = sched::tq_append_plan(n_seq, n_tok, t.g.n_kv_heads, t.g.head_dim);
+        const long long waves = p.n_grp * n_seq * t.g.n_kv_heads * p.wpr;
+        if ((waves + 3) / 4 > 0x7fffffffLL || p.n_grp > 0x7fffffffLL) return hipErrorInvalidValue;
         const dim3 gr((unsigned)((waves + 3) / 4));
 #define PI_TQ_APPEND(DD, RR, WW)                                                                            \
     hipLaunchKernelGGL((tq_append_kernel<DD, RR, WW>), gr, dim3(256), 0, s, t, k, v, page_table, max_pages, \
-                       start_pos, n_seq, n_tok, (int)n_grp)
-#define PI_TQ_APPEND_D(DD)                                     \
-    if (wpr == 1) PI_TQ_APPEND(DD, 8, 1);                      \
-    else switch (r) {                                          \
-        case 8: PI_TQ_APPEND(DD, 8, DD / 64); break;           \
-        case 4: PI_TQ_APPEND(DD, 4, DD / 64); break;           \
-        case 2: PI_TQ_APPEND(DD, 2, DD / 64); break;           \
-        default: PI_TQ_APPEND(DD, 1, DD / 64);                 \
+                       start_pos, n_seq, n_tok, (int)p.n_grp)
+        // at r 8 one wavefront a group or D / 64 of them (tq_append_plan)
+#define PI_TQ_APPEND_R(DD)                                                \
+    switch (p.r * 8 + p.wpr) {                                            \
+        case 8 * 8 + 1: PI_TQ_APPEND(DD, 8, 1); break;                    \
+        case 8 * 8 + DD / 64: PI_TQ_APPEND(DD, 8, DD / 64); break;        \
+        case 4 * 8 + 1: PI_TQ_APPEND(DD, 4, 1); break;                    \
+        case 4 * 8 + 2: PI_TQ_APPEND(DD, 4, 2); break;                    \
+        case 2 * 8 + 1: PI_TQ_APPEND(DD, 2, 1); break;                    \
+        case 2 * 8 + 2: PI_TQ_APPEND(DD, 2, 2); break;                    \
+        case 1 * 8 + 1: PI_TQ_APPEND(DD, 1, 1); break;                    \
+        case 1 * 8 + 2: PI_TQ_APPEND(DD, 1, 2); break;                    \
+        default: return hipErrorInvalidValue;                             \
     }
         if (t.g.head_dim == 128) {
-            PI_TQ_APPEND_D(128)
+            PI_TQ_APPEND_R(128)
+        } else if (p.wpr == 4 && p.r < 8) {
+            switch (p.r) {
+                case 4: PI_TQ_APPEND(256, 4, 4); break;
+                case 2: PI_TQ_APPEND(256, 2, 4); break;
+                default: PI_TQ_APPEND(256, 1, 4);
+            }
         } else {
-            PI_TQ_APPEND_D(256)
+            PI_TQ_APPEND_R(256)
         }
-#undef PI_TQ_APPEND_D
+#undef PI_TQ_APPEND_R
 #undef PI_TQ_APPEND
     } else if (t.g.head_dim < 1 || t.g.head_dim > kTqMaxDim)
         return hipErrorInvalidValue;

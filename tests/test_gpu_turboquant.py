@@ -9,6 +9,9 @@ byte.  Decode: per head row
 cache); the GPU dot uses f16 centroids (relative rounding <= 1.9e-4) and
 keeps the weights below 1e-7 that the reference's value sum skips.
 """
+import os
+import subprocess
+
 import numpy as np
 import pytest
 import torch
@@ -212,26 +215,48 @@ def test_decode_c4_shape_d256_gate(gqa_mode):
         assert err <= 1e-2, f"seq {i} (L={lens[i]}): rel err {err}"
 
 
-# groups of 1, 2, 4 and 8 tokens and unsplit groups of 8 (the row counts that pick each), starts
-# inside a group, several sequences a launch, and a launch that ends mid-group
-@pytest.mark.parametrize("d,hkv,n_tok", [(128, 2, 5), (128, 8, 270), (128, 8, 515), (128, 8, 1027), (256, 2, 515),
-                                         (256, 2, 1030), (256, 4, 1031), (128, 16, 4099), (256, 8, 4097)])
-def test_append_row_groups_bit_exact(d, hkv, n_tok):
+def _append_plan(n_seq, n_tok, hkv, d):
+    """(tokens a group, wavefronts a group) of an append launch (tests/cpp/test_tq_sched.cpp)."""
+    exe = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "_build", "test_tq_sched")
+    out = subprocess.run([exe, str(n_seq), str(n_tok), str(hkv), str(d)], capture_output=True, text=True, check=True)
+    return tuple(int(x) for x in out.stdout.split())
+
+
+# every kernel, by the (tokens, wavefronts) a group that each launch picks; starts inside a group,
+# launches that end mid-group, few sequences of many tokens and many of few
+@pytest.mark.parametrize("d,hkv,n_seq,n_tok,plan", [
+    (128, 2, 2, 5, (1, 2)), (128, 8, 2, 135, (2, 2)), (128, 8, 2, 270, (4, 2)), (128, 8, 2, 515, (8, 2)),
+    (128, 8, 1, 1027, (8, 2)), (128, 16, 1, 4099, (8, 1)), (128, 8, 512, 1, (1, 1)), (128, 8, 300, 2, (1, 1)),
+    (128, 8, 600, 3, (2, 1)), (128, 8, 300, 5, (4, 1)),
+    (256, 2, 1, 5, (1, 4)), (256, 2, 2, 270, (2, 4)), (256, 2, 2, 515, (4, 4)), (256, 2, 1, 2100, (8, 4)),
+    (256, 8, 1, 4097, (8, 1)), (256, 2, 512, 1, (1, 2)), (256, 2, 1024, 1, (1, 1)), (256, 2, 256, 3, (2, 2)),
+    (256, 2, 600, 3, (2, 1)), (256, 2, 260, 5, (4, 2)), (256, 2, 520, 5, (4, 1))])
+def test_append_row_groups_bit_exact(d, hkv, n_seq, n_tok, plan):
+    assert _append_plan(n_seq, n_tok, hkv, d) == plan
     dev = device()
-    rng = np.random.default_rng(d + n_tok)
-    starts = [3, 16] if n_tok < 1000 else [21]
+    rng = np.random.default_rng(d + n_tok + n_seq)
+    starts = np.array([21, 3, 16] * n_seq)[:n_seq]
+    if n_seq > 2:
+        starts = rng.integers(0, 33, n_seq)
     R, G = _matrices(hkv, d)
-    pages = (max(starts) + n_tok + 15) // 16
-    pt = rng.permutation(len(starts) * pages).reshape(len(starts), pages).astype(np.int32)
-    k, v = (rng.standard_normal((len(starts), n_tok, hkv, d)).astype(np.float32) for _ in range(2))
+    pages = (int(starts.max()) + n_tok + 15) // 16
+    pt = rng.permutation(n_seq * pages).reshape(n_seq, pages).astype(np.int32)
+    k, v = (rng.standard_normal((n_seq, n_tok, hkv, d)).astype(np.float32) for _ in range(2))
     pool = rt.TqPool(dev, pt.size, hkv, head_dim=d)
-    pool.append(to_dev(k), to_dev(v), to_dev(pt), to_dev(np.array(starts, np.int32)))
-    toks = sorted({0, 1, 4, min(7, n_tok - 1), n_tok - 2, n_tok - 1} | set(rng.integers(0, n_tok, 20).tolist()))
-    for i, s0 in enumerate(starts):
-        keys, norms, vals = (x.cpu().numpy() for x in pool.read(to_dev(pt), i, s0, n_tok))
-        if s0 % 16:  # the slots before the launch stay as the pool was created
-            assert not pool.read(to_dev(pt), i, 0, s0)[2].any()
+    pool.append(to_dev(k), to_dev(v), to_dev(pt), to_dev(starts.astype(np.int32)))
+    ptd = to_dev(pt)
+    toks = sorted({0, 1, 4, 7, n_tok - 2, n_tok - 1} | set(rng.integers(0, n_tok, 20).tolist()))
+    toks = [t for t in toks if 0 <= t < n_tok]
+    for i in sorted({0, 1, n_seq // 2, n_seq - 1} & set(range(n_seq))):
+        s0 = int(starts[i])
+        keys, norms, vals = (x.cpu().numpy() for x in pool.read(ptd, i, s0, n_tok))
+        # the slots around the launch's stay as the pool was created
+        if s0:
+            assert not any(x.any() for x in pool.read(ptd, i, 0, s0))
+        if s0 + n_tok < 16 * pages:
+            assert not any(x.any() for x in pool.read(ptd, i, s0 + n_tok, 16 * pages - s0 - n_tok))
         assert np.array_equal(vals, v[i].astype(np.float16))
         for t in toks:
             want, wn = o.tq_cache_append_keys(k[i, t], R, G)
             assert np.array_equal(keys[t], want[:, :keys.shape[-1]]) and np.array_equal(norms[t], wn)
+    pool.close()

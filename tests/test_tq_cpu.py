@@ -5,6 +5,9 @@ TurboQuant::new (src/turboquant/mod.rs:76-103) on the host; the device
 quantizer is only bit-compatible with the reference if these matrices are
 identical to the restatement's, bit for bit.
 """
+import os
+import subprocess
+
 import numpy as np
 import pytest
 
@@ -24,3 +27,12 @@ def test_generate_matches_oracle_bitwise(dim, seed):
 def test_generate_rejects_bad_arguments():
     with pytest.raises(rt.InvalidArg):
         rt.tq_generate(0, 1)
+
+
+def test_append_groups_host_check():
+    """tests/cpp/test_tq_sched.cpp: an append's groups cover its tokens and compute at most twice
+    their rows, whatever the number of sequences and tokens."""
+    exe = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "_build", "test_tq_sched")
+    assert os.path.exists(exe), "tests/cpp not built (python -m powerinfer_x64_amd.build)"
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout.strip().endswith("0 failures"), r.stdout + r.stderr
