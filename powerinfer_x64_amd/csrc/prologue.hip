@@ -545,7 +545,11 @@ __global__ __launch_bounds__(256) void attn_prologue_vec_kernel(
     // after them only the q heads.  A kernel of its own, without the V rows' registers (76
     // instead of 114 at EPL 4), so that the rows can be requested before the cos / sin table
     // without costing residents: 1024 tokens, 16/2 heads, D 256 12.8 -> 10.3 us; 4096, 32/8,
-    // D 128 46.4 -> 40.6.
+    // D 128 46.4 -> 40.6.  The other launches build the table first: with the rows held across
+    // it EPL 4 takes 140 registers instead of 116, three workgroups a CU instead of four (16/2
+    // heads, D 256, f16: 200 / 1024 / 4096 sequences of a token 8.1 / 19.0 / 50.8 us against
+    // 6.7 / 14.7 / 47.5, 200 of 15 tokens 35.3 against 31.1), and up to 128 tokens, where no CU is
+    // full, they time alike (4.2 .. 7.2 us at D 64, 128 and 256).
     const int toks = n_seq * n_tok;
     const int n_pg = BYPAGE ? n_seq * ppn * g.n_kv_heads : 0;
     if (BYPAGE && (int)blockIdx.x < n_pg) {
@@ -598,8 +602,10 @@ __global__ __launch_bounds__(256) void attn_prologue_vec_kernel(
         if (!BYPAGE && kn) load_vec<EPL>(kw, kn + e0);
     };
     const int hfirst = blockIdx.y * per + wv;
-    load_rows(hfirst);
-    load_weights();
+    if (BYPAGE) {
+        load_rows(hfirst);
+        load_weights();
+    }
     // cos / sin of the workgroup's token position, once per pair (every thread of the
     // workgroup works on that token)
     for (int i = threadIdx.x; i < n_pairs; i += 256) {
@@ -613,7 +619,8 @@ __global__ __launch_bounds__(256) void attn_prologue_vec_kernel(
         *sn = cs_s[1][i];
     };
     for (int head0 = hfirst; head0 < h1; head0 += 4 * MH) {
-        if (head0 != hfirst) load_rows(head0);
+        if (!BYPAGE || head0 != hfirst) load_rows(head0);
+        if (!BYPAGE && head0 == hfirst) load_weights();
 #pragma unroll
         for (int m = 0; m < MH; ++m) {
             const int head = head0 + 4 * m;
@@ -746,10 +753,14 @@ hipError_t launch_attn_prologue(float* q, float* k, const float* v, const float*
         const long long n_pg = by_page ? (long long)n_seq * ppn * g.n_kv_heads : 0;
         if (toks + n_pg > 0x7fffffffLL) return hipErrorInvalidValue;
         // Head groups (y) per token: each builds its token's cos / sin table again, so only as
-        // many as fill the chip once (about 1024 resident workgroups); more cost a
-        // 1000-token prompt 40.7 us instead of 22.1 (f32 pool, 32/32 heads, D 128) and 18.6
-        // instead of 9.8 (f16, 32/8, D 64), fewer a 256-token one 9.6 instead of 7.9 (f16,
-        // 32/8, D 128).
+        // many as keep the launch at about 1024 workgroups (four a CU, what fits at once where
+        // registers are short).  A group per four heads cost a 1000-token prompt 40.7 us instead
+        // of 22.1 (f32 pool, 32/32 heads, D 128) and 18.6 instead of 9.8 (f16, 32/8, D 64), 512
+        // sequences of one token 16.5 instead of 13.4 (32/8, D 128) and 12.2 instead of 9.4
+        // (16/2, D 256); fewer groups a 256-token prompt 9.6 instead of 7.9 (f16, 32/8, D 128).
+        // A tuned value: 768 and 1536 took 0.9 to 1.3 of its time over 1 to 4096 tokens, but for 64
+        // sequences of 8 tokens, where one group a token (and with it the XCD order above) takes
+        // 0.6 to 0.95 (f32, 32/32 heads, D 128: 27.7 against 44.5 us).
         const int split_heads = by_page ? n_q_heads : heads;
         const unsigned gy = (unsigned)std::max<long long>(1, std::min<long long>((split_heads + 3) / 4, 1024 / toks));
         const dim3 grid_v((unsigned)(toks + n_pg), gy);
