@@ -27,6 +27,7 @@
 
 #include "pi_device.hpp"
 #include "pi_launch.hpp"
+#include "prefill_loads.hpp"
 
 namespace pi {
 namespace {
@@ -154,11 +155,6 @@ __device__ __forceinline__ float max32(const f32x16& s, const f32x16& t) {
 // registers at 32 query rows, so the workgroup has 4 wavefronts (one per SIMD,
 // up to 512 registers each) and two unit buffers; each wavefront runs its MFMA
 // and softmax phases back to back.
-template <int D> struct PrefillCfg;
-template <> struct PrefillCfg<64> { static constexpr int NW = 8, NB = 4; };
-template <> struct PrefillCfg<128> { static constexpr int NW = 8, NB = 4; };
-template <> struct PrefillCfg<256> { static constexpr int NW = 4, NB = 2; };
-
 template <typename T, int HPW, int D, bool PG>
 __global__ __launch_bounds__(64 * PrefillCfg<D>::NW, 1) void prefill_fa_kernel(PrefillArgs a) {
     typedef typename Mfma<T>::v8 v8;
@@ -169,14 +165,10 @@ __global__ __launch_bounds__(64 * PrefillCfg<D>::NW, 1) void prefill_fa_kernel(P
     constexpr int WROWS = ROWS * RT;  // query rows per workgroup
     constexpr int NB = PrefillCfg<D>::NB;  // unit buffers
     constexpr int NDT = D / 32;       // 32-dim tiles of O^T
-    constexpr int KS = D + 8;         // K [key][dim] row stride (elements): 16 bytes of padding
-    constexpr int KCH = KS / 8;       // 16-byte chunks per K row (17 or 33)
-    // direct loads of 1 KB per K tile: 17 or 33 padded rows; paged, D / 8 (one per 16-byte chunk)
-    constexpr int K_INSTR = PG ? D / 8 : BN * KCH / 64;
-    constexpr int KJ = (K_INSTR + NW - 1) / NW;  // K loads per wavefront
-    constexpr int V_INSTR = BN * D * 2 / 1024;  // direct loads of 1 KB per V tile (16 or 32)
-    constexpr int VJ = V_INSTR / NW;  // V loads per wavefront
-    constexpr int VRPI = 1024 / (2 * D);  // V rows per load (4 or 2)
+    typedef PrefillLoads<D, PG> LD;
+    constexpr int KS = LD::KS, KCH = LD::KCH, K_INSTR = LD::K_INSTR, KJ = LD::KJ, VJ = LD::VJ;
+    static_assert(LD::BN == BN, "tile");
+    constexpr int VRPI = 1024 / (2 * D);  // V rows per load (8, 4 or 2)
     constexpr int VCPR = D / 8;       // 16-byte chunks per V row (8, 16 or 32)
     // contiguous V rows: the 32-dim group of a chunk is XORed with the row's low bits (two
     // at D >= 128, one at D = 64, whose rows hold two groups)
@@ -407,7 +399,7 @@ __global__ __launch_bounds__(64 * PrefillCfg<D>::NW, 1) void prefill_fa_kernel(P
     // lag partner's share) after its softmax, when its lag partner runs its MFMA phase; the
     // lag waves then issue none and their path through a step (softmax, MFMA phase) is free
     // of load issue, which stalls on the direct-load path's latency.
-    constexpr int LPD = (PG && NW == 8) ? 2 : 1;  // load passes of a loading wave
+    constexpr int LPD = LD::LPD;  // load passes of a loading wave
     const bool loader = wave < NW / LPD;
     // this wave's page ids for the K tile of the unit issued last (the next unit's V tile)
     unsigned koff_prev[LPD][KJ] = {};
@@ -640,24 +632,20 @@ __global__ __launch_bounds__(64 * PrefillCfg<D>::NW, 1) void prefill_fa_kernel(P
         __builtin_amdgcn_s_setprio(0);
     };
     if constexpr (NW == 8) {
-        // this wave's loads per unit (K + V): 5 for wave 0 and 4 for the others with the
-        // padded contiguous K tile (17 loads); from the pool D / 16 for a lead wave and none
-        // for a lag wave
-        constexpr int NLP = LPD * ((K_INSTR / NW) + VJ);
-        const int nl = PG ? NLP : (wave == 0 ? 3 : 2) + 2;
         // Wait until this wave's loads of unit u are complete while its loads of
-        // the next `ahead` units (0, 1 or 2) may still be in flight.
+        // the next `ahead` units (0, 1 or 2) may still be in flight: N0 of them per unit by
+        // wave 0, which has the odd K load of the padded rows, N1 by the others (from the pool
+        // by the lead waves; the lag waves have none, and wait for none).
         // vmcnt(n) on gfx9: bits 3:0 and 15:14; expcnt 6:4 = 7; lgkmcnt 11:8 = 15
 #define PI_VMCNT(n) __builtin_amdgcn_s_waitcnt(0x0F70 | ((n) & 15) | (((n) >> 4) << 14))
+        constexpr int N0 = LD::unit_loads(0), N1 = LD::unit_loads(1);
         auto wait_unit = [&](int ahead) {
             if (ahead == 2) {
-                if (PG) PI_VMCNT(2 * NLP);
-                else if (nl == 5) PI_VMCNT(10);
-                else PI_VMCNT(8);
+                if (N0 != N1 && wave == 0) PI_VMCNT(2 * N0);
+                else PI_VMCNT(2 * N1);
             } else if (ahead == 1) {
-                if (PG) PI_VMCNT(NLP);
-                else if (nl == 5) PI_VMCNT(5);
-                else PI_VMCNT(4);
+                if (N0 != N1 && wave == 0) PI_VMCNT(N0);
+                else PI_VMCNT(N1);
             } else {
                 PI_VMCNT(0);
             }
