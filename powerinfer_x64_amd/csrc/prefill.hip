@@ -76,6 +76,9 @@ struct PrefillArgs {
     // every workgroup walks nqb + 1 key tiles and one wave of workgroups fills
     // the chip evenly (else: one block each, heaviest first)
     int paired;
+    // contiguous source: grid y = sequence, z = query block instead of y = query block, z =
+    // (sequence, split); launch_d's choice
+    int seq_fast;
     // key split (a launch with fewer workgroups than CUs): blockIdx.z = batch * ksplit +
     // split.  A query block of n <= kthr key tiles is not split: split 0 takes all its
     // tiles and writes the output, the other splits skip it.  A longer one runs in
@@ -192,7 +195,7 @@ __global__ __launch_bounds__(64 * PrefillCfg<D>::NW, 1) void prefill_fa_kernel(P
     }
     const int nqb = (a.S + WROWS - 1) / WROWS;
     int by = blockIdx.y, bz = blockIdx.z;
-    if (!PG && a.ksplit == 1) {  // launch_d's grid order
+    if (!PG && a.seq_fast) {
         by = blockIdx.z;
         bz = blockIdx.y;
     }
@@ -818,7 +821,7 @@ __global__ __launch_bounds__(512, 1) void prefill_fa256_kernel(PrefillArgs a) {
     }
     const int nqb = (a.S + WROWS - 1) / WROWS;
     int by = blockIdx.y, bz = blockIdx.z;
-    if (!PG && a.ksplit == 1) {  // launch_d's grid order
+    if (!PG && a.seq_fast) {
         by = blockIdx.z;
         bz = blockIdx.y;
     }
@@ -1896,19 +1899,29 @@ bool use_fa256() {
 }
 
 template <int D>
-void launch_d(const PrefillArgs& a, int hpw, int n_kv_heads, int seq_len, int batch, bool bf,
+void launch_d(PrefillArgs a, int hpw, int n_kv_heads, int seq_len, int batch, bool bf,
               hipStream_t s) {
     constexpr int NW = PrefillCfg<D>::NW;
-    // x = workgroup's head set (fastest), y = sequence, z = query block (reversed in the
-    // kernel, so the heaviest blocks of all sequences go first: 4 prompts of 777 tokens,
-    // 32/8 heads, D 64 39.6 -> 33.2 us against the sequence slowest); with x = KV head and
-    // round-robin dispatch over the 8 XCDs, a KV head's K/V stays in one L2.
-    // A key split keeps y = query block, z = (sequence, split): the splits of a block
-    // next to each other ran 1000 tokens at D 128 in 40.5 us instead of 33.9.
+    // x = workgroup's head set, fastest: workgroups are dispatched round-robin over the 8 XCDs,
+    // so with 8 or a multiple of it a head set's K / V stays in one L2.  Next the query block
+    // (reversed in the kernel, the heaviest first) or, seq_fast, the sequence:
+    // - single causal blocks, so that the heaviest of all sequences go first: 4 prompts of 777
+    //   tokens, 32/8 heads 36.6 -> 30.3 us at D 64, 46.8 -> 42.3 at D 128; 0.96 of the time over 47
+    //   batches of 2 to 32 prompts (0.74 to 1.03);
+    // - other numbers of head sets, each of which then runs on fewer XCDs: 0.98 over 38 paired and
+    //   non-causal batches at 2 or 4 head sets (0.81 to 1.02; 16 x 512, 16/2 heads, D 64, not
+    //   causal 46.6 -> 37.5 us).
+    // Equal blocks (paired or not causal) of 8 or 32 head sets go sequence by sequence: with all
+    // sequences' K / V in each L2 at once they took 1.005 of the time over 104 batches (0.92 to
+    // 1.09; 4 x 4096, 32/32 heads, D 128, not causal 1016 -> 1098 us; 16 x 512, 32/8, D 64, paired
+    // 49.5 -> 53.5).
+    // A key split keeps y = query block too: the splits of a block next to each other ran 1000
+    // tokens at D 128 in 40.5 us instead of 33.9.
     const int rows = ROWS * NW / hpw;
     const int nqb = (seq_len + rows - 1) / rows;
     const unsigned gx = n_kv_heads * (a.group / hpw), blocks = a.paired ? (nqb + 1) / 2 : nqb;
-    const dim3 grid = a.ksplit > 1 ? dim3(gx, blocks, batch * a.ksplit) : dim3(gx, batch, blocks);
+    a.seq_fast = a.ksplit == 1 && ((a.causal && !a.paired) || gx % 8 != 0);
+    const dim3 grid = a.seq_fast ? dim3(gx, batch, blocks) : dim3(gx, blocks, batch * a.ksplit);
     const dim3 block(64 * NW);
     if constexpr (D == 256) {
         if (use_fa256()) {  // same grid: 128 / hpw query rows per workgroup either way

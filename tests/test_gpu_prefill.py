@@ -321,3 +321,26 @@ def test_prefill_many_prompts_repeat_bit_exact(d):
     for i, row in ((0, s - 1), (5, 400), (b - 1, s - 1)):
         ref = ref64.attention(qn[i, row], kn[i, :row + 1], vn[i, :row + 1], lambda h: h % hkv)
         assert row_rel_err(first[i, row].cpu().numpy(), ref) <= 1e-2
+
+
+@pytest.mark.parametrize("causal,paired", [(True, "0"), (True, "1"), (False, "0")])
+@pytest.mark.parametrize("d,hq,hkv,s", [(64, 32, 8, 600), (128, 8, 8, 520), (256, 16, 8, 130), (128, 12, 4, 300)])
+def test_prefill_grid_orders(monkeypatch, d, hq, hkv, s, causal, paired):
+    """The launch orders (sequence by sequence, or the sequences interleaved: by the number of
+    head sets, 8 or a multiple of it or not, and the schedule) against each prompt alone: bit for
+    bit, and one row against the oracle's formula."""
+    from powerinfer_x64_amd import runtime as rt
+    dev = device()
+    monkeypatch.setenv("PI_PREFILL_PAIRED", paired)
+    monkeypatch.setenv("PI_PREFILL_KSPLIT", "1")
+    rng = np.random.default_rng(d + s + hq)
+    x = [rng.standard_normal((3, s, h, d)).astype(np.float32) for h in (hq, hkv, hkv)]
+    q, k, v = (to_dev(a, torch.float16) for a in x)
+    out = rt.attn_prefill(dev, q, k, v, causal=causal)
+    for i in range(3):
+        one = rt.attn_prefill(dev, *(t[i:i + 1].contiguous() for t in (q, k, v)), causal=causal)
+        assert torch.equal(out[i], one[0])
+    n = s - 1 if causal else s
+    ref = ref64.attention(*(t[2].float().cpu().numpy()[sl] for t, sl in ((q, n - 1), (k, slice(n)), (v, slice(n)))),
+                          lambda h: h % hkv)
+    assert row_rel_err(out[2, n - 1].cpu().numpy(), ref) <= 1e-2
