@@ -226,40 +226,34 @@ __global__ __launch_bounds__(256) void gdn_rmsnorm_gated_kernel(float* __restric
     }
 }
 
-// The same at V = 64, 128 or 256 and 16-byte aligned rows: V / 4 lanes a row, so a wavefront
-// loads 256 / V rows with one 16-byte access per lane, and each wavefront takes NR such
-// groups, all requested before any is used: 4096 tokens x 32 heads x 128 (201 MB) in 31 us
-// (6.5 TB/s; 47 with one row and 8 bytes a lane per wavefront).
-template <int V>
+// The same at V = 64, 128 or 256 and rows aligned to E values (16 or 8 bytes): V / E lanes a row,
+// 64 E / V rows a wavefront, one access per lane.  Bound by memory: 4096 tokens x 32 heads x 128
+// (201 MB) in 30 us at E 4 (6.7 TB/s) and 34.5 at E 2, where the any-width kernel takes 42; 64 x
+// 32 rows 2.6 us.  Two such groups a wavefront, all requested before any is used, took 30.5 and
+// 2.9 us, and 8.1 instead of 7.0 at 1024 x 32: half the wavefronts hide less latency than the
+// second load in flight.
+template <int V, int E>
 __global__ __launch_bounds__(256) void gdn_rmsnorm_gated_vec_kernel(float* __restrict__ o,
                                                                     const float* __restrict__ z,
                                                                     const float* __restrict__ w,
                                                                     int n_rows, float eps) {
-    constexpr int LPR = V / 4, NR = 2;
-    const int lane = threadIdx.x & 63, c = 4 * (lane % LPR);
-    const int first = ((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6)) * NR * (64 / LPR) + lane / LPR;
-    f32x4 ov[NR], zv[NR];
+    typedef float fe __attribute__((ext_vector_type(E)));
+    constexpr int LPR = V / E;
+    const int lane = threadIdx.x & 63, c = E * (lane % LPR);
+    const int row = ((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6)) * (64 / LPR) + lane / LPR;
+    const size_t at = (size_t)min(row, n_rows - 1) * V + c;
+    const fe ov = *reinterpret_cast<const fe*>(o + at), zv = *reinterpret_cast<const fe*>(z + at);
+    const fe wv = *reinterpret_cast<const fe*>(w + c);
+    float ss = 0.f;
 #pragma unroll
-    for (int i = 0; i < NR; ++i) {
-        const size_t at = (size_t)min(first + i * (64 / LPR), n_rows - 1) * V + c;
-        ov[i] = *reinterpret_cast<const f32x4*>(o + at);
-        zv[i] = *reinterpret_cast<const f32x4*>(z + at);
-    }
-    const f32x4 wv = *reinterpret_cast<const f32x4*>(w + c);
+    for (int e = 0; e < E; ++e) ss += ov[e] * ov[e];
 #pragma unroll
-    for (int i = 0; i < NR; ++i) {
-        const int row = first + i * (64 / LPR);
-        float ss = 0.f;
+    for (int m = LPR / 2; m >= 1; m >>= 1) ss = wave_sum_xor(ss, m);
+    const float scale = 1.0f / sqrtf(ss / (float)V + eps);
+    fe r;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) ss += ov[i][e] * ov[i][e];
-#pragma unroll
-        for (int m = LPR / 2; m >= 1; m >>= 1) ss = wave_sum_xor(ss, m);
-        const float scale = 1.0f / sqrtf(ss / (float)V + eps);
-        f32x4 r;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = (ov[i][e] * scale * wv[e]) * (zv[i][e] / (1.0f + expf(-zv[i][e])));
-        if (row < n_rows) *reinterpret_cast<f32x4*>(o + (size_t)row * V + c) = r;
-    }
+    for (int e = 0; e < E; ++e) r[e] = (ov[e] * scale * wv[e]) * (zv[e] / (1.0f + expf(-zv[e])));
+    if (row < n_rows) *reinterpret_cast<fe*>(o + at) = r;
 }
 
 // Decode step.  A workgroup owns (sequence, V head, 32 state columns): a
@@ -1464,14 +1458,20 @@ hipError_t launch_gdn_conv_state(const float* x, float* state, int32_t n_tok, in
 hipError_t launch_gdn_rmsnorm_gated(float* o, const float* z, const float* w, int32_t n_rows,
                                     int32_t n_v_heads, int32_t v_hd, float eps, hipStream_t s) {
     const int n = n_rows * n_v_heads;
-    if ((v_hd == 64 || v_hd == 128 || v_hd == 256) && (((uintptr_t)o | (uintptr_t)z | (uintptr_t)w) & 15) == 0) {
-        const int per = 4 * 2 * (256 / v_hd);  // rows a workgroup
-        const dim3 grid((unsigned)((n + per - 1) / per));
-        if (v_hd == 64) hipLaunchKernelGGL(gdn_rmsnorm_gated_vec_kernel<64>, grid, dim3(256), 0, s, o, z, w, n, eps);
-        else if (v_hd == 128) hipLaunchKernelGGL(gdn_rmsnorm_gated_vec_kernel<128>, grid, dim3(256), 0, s, o, z, w, n, eps);
-        else hipLaunchKernelGGL(gdn_rmsnorm_gated_vec_kernel<256>, grid, dim3(256), 0, s, o, z, w, n, eps);
-        return hipGetLastError();
+    const uintptr_t low = (uintptr_t)o | (uintptr_t)z | (uintptr_t)w;
+#define PI_NORM_VEC(V, E)                                                                              \
+    if (v_hd == V && low % (4 * E) == 0) {                                                             \
+        constexpr int per = 4 * 64 * E / V; /* rows a workgroup */                                     \
+        hipLaunchKernelGGL((gdn_rmsnorm_gated_vec_kernel<V, E>), dim3((unsigned)(((long long)n + per - 1) / per)), \
+                           dim3(256), 0, s, o, z, w, n, eps);                                          \
+        return hipGetLastError();                                                                      \
     }
+    PI_NORM_VEC(64, 4)
+    PI_NORM_VEC(128, 4)
+    PI_NORM_VEC(256, 4)
+    PI_NORM_VEC(64, 2)
+    PI_NORM_VEC(128, 2)
+#undef PI_NORM_VEC
     hipLaunchKernelGGL(gdn_rmsnorm_gated_kernel, dim3((n + 3) / 4), dim3(256), 0, s, o, z, w, n,
                        v_hd, eps);
     return hipGetLastError();

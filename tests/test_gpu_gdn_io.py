@@ -90,6 +90,34 @@ def test_rmsnorm_gated_matches_oracle():
     np.testing.assert_allclose(to.cpu().numpy(), ref, rtol=2e-5, atol=2e-6)
 
 
+@pytest.mark.parametrize("rows,hv,dv", [(1, 1, 64), (5, 3, 64), (1, 3, 128), (33, 2, 128), (1, 1, 256), (7, 5, 256), (3, 5, 96)])
+@pytest.mark.parametrize("off", [0, 1, 2, 3])
+def test_rmsnorm_gated_alignments(rows, hv, dv, off):
+    """The 16-byte, 8-byte and any-width kernels, by the alignment of o, z and w together, at row
+    counts beside a wavefront's and a workgroup's rows; nothing around the rows is written.  f32
+    throughout: a sum of dv squares in another order, 2^-24 dv relative at most, and a few rounded
+    products and an exponential (2^-22 each)."""
+    from powerinfer_x64_amd import runtime as rt
+    dev = device()
+    rng = np.random.default_rng(rows + dv + off)
+    n = rows * hv * dv
+    o, z = (rng.standard_normal((rows, hv, dv)).astype(np.float32) for _ in range(2))
+    w = rng.uniform(0.5, 1.5, dv).astype(np.float32)
+    ref = orc.rmsnorm_gated(o, z, w, 1e-6)
+    for who in ("o", "z", "w"):
+        buf = torch.full((n + 8,), 7.0, device="cuda")
+        at = {k: off if k == who else 0 for k in "ozw"}
+        to = buf[at["o"]:at["o"] + n].view(rows, hv, dv)
+        to.copy_(to_dev(o))
+        tz = torch.empty(n + 8, device="cuda")[at["z"]:at["z"] + n].view(rows, hv, dv)
+        tz.copy_(to_dev(z))
+        tw = torch.empty(dv + 8, device="cuda")[at["w"]:at["w"] + dv]
+        tw.copy_(to_dev(w))
+        rt.gdn_rmsnorm_gated(dev, to, tz, tw, 1e-6)
+        assert float(np.abs(to.cpu().numpy() - ref).max()) <= (2.0 ** -24 * dv + 2.0 ** -20) * float(np.abs(ref).max())
+        assert bool((buf[:at["o"]] == 7).all()) and bool((buf[at["o"] + n:] == 7).all())
+
+
 def test_gdn_layer_body_prefill_then_decode():
     """conv1d -> split q/k/v -> gates -> recurrence -> RMSNormGated for a 200-token
     prompt and 3 decode tokens, all on the GPU, against the oracle's per-token
