@@ -1576,13 +1576,14 @@ static int gdn_layer_step(pi_handle h, pi_gdn_layer L, const float* dx, const fl
     }
     const size_t n = (size_t)n_tokens, C = L->conv_dim, kd = (size_t)L->hk * L->dk;
     const size_t vd = (size_t)L->hv * L->dv, nh = (size_t)L->hv;
-    // activation, q, k, v, beta, g
-    const size_t need = n * C + 2 * n * kd + n * vd + 2 * n * nh;
+    const bool split_conv = n > 1 && pi::gdn_layer_in_ok(dx, L->d_conv_state, L->hk, L->hv, L->dk, L->dv, L->d_conv);
+    // the separate conv's activation rows, then q, k, v (for one token its row holds them), beta, g
+    const size_t act_f = split_conv ? 0 : n * C, need = act_f + (n > 1 ? n * C : 0) + 2 * n * nh;
     int rc = grow(h, &L->d_buf, &L->buf_floats, need, s, "gdn layer staging", false);
     if (rc) return rc;
-    float *act = L->d_buf, *dq = act + n * C, *dk = dq + n * kd, *dv = dk + n * kd;
+    float *act = L->d_buf, *dq = n > 1 ? act + act_f : act, *dk = dq + n * kd, *dv = dk + n * kd;
     float *db = dv + n * vd, *dg = db + n * nh;
-    if (n > 1 && pi::gdn_layer_in_ok(dx, L->d_conv_state, L->hk, L->hv, L->dk, L->dv, L->d_conv)) {
+    if (split_conv) {
         // conv, split and gates in one launch, then the recurrence, which rolls the conv state
         PI_HIP(h, pi::launch_gdn_layer_in(dx, L->d_conv_state, L->d_w, dbr, dar, L->d_ssm_a, L->d_dt, dq, dk, dv,
                                           db, dg, n_tokens, L->hk, L->hv, L->dk, L->dv, s),
@@ -1599,11 +1600,7 @@ static int gdn_layer_step(pi_handle h, pi_gdn_layer L, const float* dx, const fl
     }
     if ((rc = pi_gdn_conv1d(h, dx, L->d_conv_state, L->d_w, act, 1, n_tokens, (int32_t)C, L->d_conv, sv)))
         return rc;
-    if (n == 1) {  // one token's row already holds q, k and v back to back
-        dq = act;
-        dk = act + kd;
-        dv = act + 2 * kd;
-    } else {
+    if (n > 1) {
         PI_HIP(h, hipMemcpy2DAsync(dq, kd * 4, act, C * 4, kd * 4, n, hipMemcpyDeviceToDevice, s), "gdn layer");
         PI_HIP(h, hipMemcpy2DAsync(dk, kd * 4, act + kd, C * 4, kd * 4, n, hipMemcpyDeviceToDevice, s), "gdn layer");
         PI_HIP(h, hipMemcpy2DAsync(dv, vd * 4, act + 2 * kd, C * 4, vd * 4, n, hipMemcpyDeviceToDevice, s), "gdn layer");

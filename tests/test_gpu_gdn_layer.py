@@ -212,3 +212,28 @@ def test_layer_prompts_equal_the_separate_steps(hk, hv, dk, dv, lens):
         buf = x.reshape(-1)
         out = layers[1].forward_dev(x, z, br, ar, buf[:n * hv * dv].view(n, hv, dv))
         assert torch.equal(out, ref)
+
+
+def test_layer_prompt_staging_holds_no_unused_rows():
+    """A layer prompt stages q, k, v and the gates and nothing else: no second set of the conv's
+    rows, which the split launch never writes (84 MB for these 2048 tokens)."""
+    from powerinfer_x64_amd import runtime as rt
+    dev = device()
+    hk, hv, d, n = 16, 32, 128, 2048
+    conv = 2 * hk * d + hv * d
+    rng = np.random.default_rng(5)
+    f = lambda *s: rng.standard_normal(s).astype(np.float32)  # noqa: E731
+    w = (f(conv, 4) * 0.5, -np.abs(f(hv)), f(hv) * 0.1, rng.uniform(0.5, 1.5, d).astype(np.float32))
+    x, z, br, ar = (to_dev(f(*s)) for s in ((n, conv), (n, hv, d), (n, hv), (n, hv)))
+    out = torch.empty((n, hv, d), device="cuda")
+    warm, layer = (rt.GdnLayer(dev, hk, hv, d, d, *w, 1e-6) for _ in range(2))
+    warm.forward_dev(x, z, br, ar, out)  # the handle's own workspace
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    layer.forward_dev(x, z, br, ar, out)
+    torch.cuda.synchronize()
+    used = before - torch.cuda.mem_get_info()[0]
+    staged = 4 * n * (conv + 2 * hv)
+    assert staged <= used <= 1.25 * staged + (8 << 20), f"{used} bytes for {staged}"
+    warm.close()
+    layer.close()
