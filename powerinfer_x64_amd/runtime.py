@@ -62,7 +62,7 @@ def _need(t: torch.Tensor, name: str, dtype=None, shape=None, dev=None):
         raise InvalidArg(f"{name}: on {t.device}, expected {dev}")
     if dtype is not None and t.dtype != dtype:
         raise InvalidArg(f"{name}: dtype {t.dtype}, expected {dtype}")
-    if shape is not None and t.shape != shape:  # a tuple or torch.Size
+    if shape is not None and t.shape != tuple(shape):
         raise InvalidArg(f"{name}: shape {tuple(t.shape)}, expected {tuple(shape)}")
     if not t.is_contiguous():
         raise InvalidArg(f"{name}: must be contiguous")

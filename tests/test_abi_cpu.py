@@ -97,3 +97,15 @@ def test_compute_imrope_freqs_host_export_matches_oracle(orc):
         ref = orc.compute_imrope_freqs(base, n_rot, list(sec))
         assert np.array_equal(out, ref)
     assert lib.pi_compute_imrope_freqs(1e4, 512, s, out.ctypes.data_as(ctypes.c_void_p)) == 5
+
+
+@pytest.mark.parametrize("shape", [(2, 3), [2, 3]])
+def test_argument_check_takes_any_shape_sequence(shape):
+    """The front end's argument check compares shapes by value, whatever sequence names them."""
+    import torch
+
+    from powerinfer_x64_amd import runtime as rt
+    rt._need(torch.zeros(2, 3), "x", torch.float32, shape)
+    rt._need(torch.zeros(2, 3), "x", torch.float32, torch.Size(shape))
+    with pytest.raises(rt.InvalidArg):
+        rt._need(torch.zeros(3, 2), "x", torch.float32, shape)
