@@ -251,3 +251,16 @@ def test_workspace_ordered_across_streams():
     torch.cuda.synchronize()
     for r, o in zip(ref, outs):
         assert all(torch.equal(r, x) for x in o)
+
+
+def test_stream_handle_with_and_without_the_raw_lookup(monkeypatch):
+    """stream() is torch's current stream, the default one and a side one, also when torch lacks
+    the lookup that skips the Stream object."""
+    from powerinfer_x64_amd import runtime as rt
+    dev = device()
+    side = torch.cuda.Stream()
+    for raw in (rt._raw_stream, None):
+        monkeypatch.setattr(rt, "_raw_stream", raw)
+        assert dev.stream() == torch.cuda.current_stream().cuda_stream
+        with torch.cuda.stream(side):
+            assert dev.stream() == side.cuda_stream
