@@ -46,11 +46,38 @@ def test_f32_prefill_tile_edges(prev, n, hq, hkv, d):
 
 @pytest.mark.parametrize("d", [64, 128, 256])
 def test_f32_prefill_max_rises_late(d):
-    """Scores that outgrow the running max tile after tile (the kernels raise it lazily)."""
+    """Scores that outgrow the running max tile after tile."""
     c = Chunk(np.random.default_rng(d), 0, 200, 4, 2, d)
     c.k *= np.linspace(0.2, 4.0, 200, dtype=np.float32)[:, None, None]
     out = c.gpu(device(), pool_dtype=torch.float32)
     _check(c, out, [0, 31, 63, 64, 130, 199])
+
+
+@pytest.mark.parametrize("late", [70, 150, 190])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_f32_prefill_largest_weight_is_exact(d, late):
+    """One key ahead of two in the first tile (one a key half) by less than 2^8, the rest far
+    behind: its weight is exactly 1 in the products too.  Scores and values are exact here, so
+    what is left is the rounding of the scaled scores below 8 (2^-22 each), an exponential, the
+    sum of three and the division (2^-23 each): 2^-20; a weight kept as bf16 hi + lo is off by
+    up to 2^-17."""
+    from powerinfer_x64_amd import runtime as rt
+    dev = device()
+    n, prev = 45, 200
+    a = 1 + np.arange(n) / 128.0  # 8 bits
+    q, k, v = np.zeros((n, 2, d), np.float32), np.zeros((1, prev + n, 1, d), np.float32), np.zeros((1, prev + n, 1, d), np.float32)
+    q[:, :, 0] = a[:, None]
+    k[0, :, 0, 0] = -64
+    k[0, [5, 40], 0, 0] = 0
+    k[0, late, 0, 0] = 4
+    v[0, late] = 1
+    pages = (prev + n + 15) // 16
+    pt = to_dev(np.random.default_rng(d).permutation(pages).astype(np.int32)[None])
+    pool = rt.KvPool(dev, pages, 1, d, dtype=torch.float32)
+    pool.append(to_dev(k), to_dev(v), pt, torch.zeros(1, dtype=torch.int32, device="cuda"))
+    out = rt.attn_prefill_paged(dev, to_dev(q), pool, pt[0].contiguous(), prev, scale=1.0).cpu().numpy()
+    w = np.exp(4 * a)
+    assert float(np.abs(out / (w / (w + 2))[:, None, None] - 1).max()) <= 2.0 ** -20
 
 
 # history, chunk and the pages made invalid: inside and at the edges of the 32-key halves and the
