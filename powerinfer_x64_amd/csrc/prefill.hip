@@ -1266,7 +1266,7 @@ __global__ __launch_bounds__(512, 1) void prefill_fa256_kernel(PrefillArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// prefill_f32_kernel / prefill_f32_256_kernel: causal attention of a chunk of
+// prefill_f32_kernel / prefill_f32_16_kernel: causal attention of a chunk of
 // queries (f32 rows) over an f32 KV pool, read through the sequence's page table
 // (src/model/mod.rs:668 token loop over :1140-1190 with an f32 cache).  Products
 // keep f32 accuracy on the bf16 MFMA by splitting each f32 operand into bf16
@@ -1629,12 +1629,13 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_kernel(PrefillArgs a) {
         }
 }
 
-// Head dim 256, v_mfma_f32_16x16x32_bf16: 32-row operands would take 256 registers for O and
-// Q^T alone.  Wavefront w owns 16 rows of head slot w / (8 / HPW) and attends whole tiles of
-// 32 keys (two buffers of a 64-key tile would need 256 KB).
-template <int HPW>
-__global__ __launch_bounds__(512, 2) void prefill_f32_256_kernel(PrefillArgs a) {
-    constexpr int D = 256, TK = 32;
+// v_mfma_f32_16x16x32_bf16.  Head dim 256, where 32-row operands would take 256 registers for O
+// and Q^T alone (and two buffers of a 64-key tile 256 KB), and short sequences at any head dim
+// (f32_sched).  Wavefront w owns 16 rows of head slot w / (8 / HPW) and attends whole tiles of
+// 32 keys.
+template <int D, int HPW>
+__global__ __launch_bounds__(512, 2) void prefill_f32_16_kernel(PrefillArgs a) {
+    constexpr int TK = 32;
     constexpr int RW = 8 / HPW;               // row tiles of 16 per workgroup
     constexpr int WROWS = 16 * RW;            // query rows per workgroup
     constexpr int NKB = TK / 16;
@@ -2207,7 +2208,17 @@ hipError_t launch_prefill_pool(const KvGeom& g, const void* q, int32_t q_f32, co
 namespace {
 struct F32Sched {
     int hpw, wrows, ksplit, kthr, q0;  // q0: first query row of a split block
+    bool rows16;                       // prefill_f32_16_kernel
 };
+
+// Sequences of up to this many keys run prefill_f32_16_kernel, one head a workgroup: half the
+// keys to load and split before the first product, no exchange of key halves, and few enough
+// rows a CU that their scattered loads and stores do not queue.  32/8 heads, D 128: 24 fresh
+// tokens 5.4 us (10.2 in 32-row blocks of 4 heads), 64 7.9 (12.3), 24 after 50 8.3 (14.4), 128
+// 13.1 (15.4); D 64 4.5 (6.9), 6.0 (7.7), 6.5 (9.1), 9.2 (9.7); D 256, 16/2 heads 7.6 (11.8),
+// 11.9 (15.9), 12.2 (17.7), 20.9 (21.3).  Past it the 32-row kernel wins at D 64 first: 64 after
+// 300 tokens 16.9 against 16.4, 128 after 100 13.2 against 13.9, 1000 37.7 against 46.9.
+constexpr int kF32ShortKeys = 128;
 
 // The f32 prefill's key split.  One workgroup (a block of wrows rows) runs on a CU at a time,
 // about 3 us a 64-key tile, so a launch with fewer blocks than CUs takes its longest block's
@@ -2218,11 +2229,13 @@ struct F32Sched {
 // fills the CUs runs whole: pieces of the average CU's tiles ran 1000 tokens at 32/32 heads,
 // D 128 in 87.6 us against 84.5.  PI_PREFILL_KSPLIT=n forces the pieces of the longest block
 // (1: none).
-F32Sched f32_sched(int q_off, int n_tok, int n_q_heads, int n_kv_heads) {
+F32Sched f32_sched(int q_off, int n_tok, int n_q_heads, int n_kv_heads, int head_dim) {
     F32Sched sc;
+    const bool is_short = (long long)q_off + n_tok <= kF32ShortKeys;
+    sc.rows16 = head_dim == 256 || is_short;
     const bool multiple = n_q_heads % n_kv_heads == 0;
     const int group = (n_q_heads + n_kv_heads - 1) / n_kv_heads;
-    sc.hpw = !multiple ? 1 : group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1);
+    sc.hpw = !multiple || is_short ? 1 : group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1);
     sc.wrows = 128 / sc.hpw;
     sc.ksplit = 1;
     sc.kthr = 0;
@@ -2269,7 +2282,7 @@ F32Sched f32_sched(int q_off, int n_tok, int n_q_heads, int n_kv_heads) {
 size_t prefill_f32_ws_floats(int32_t q_off, int32_t n_tok, int32_t n_q_heads, int32_t n_kv_heads,
                              int32_t head_dim) {
     if (q_off < 0 || n_tok <= 0 || n_q_heads <= 0 || n_kv_heads <= 0) return 0;
-    const F32Sched sc = f32_sched(q_off, n_tok, n_q_heads, n_kv_heads);
+    const F32Sched sc = f32_sched(q_off, n_tok, n_q_heads, n_kv_heads, head_dim);
     return sc.ksplit > 1 ? (size_t)sc.ksplit * n_tok * n_q_heads * (head_dim + 2) : 0;
 }
 
@@ -2305,7 +2318,7 @@ hipError_t launch_prefill_f32(const KvGeom& g, const float* q, const int32_t* pa
     a.vstride = g.vstride;
     a.n_pages = g.n_pages;
     a.ksplit = 1;
-    F32Sched sc = f32_sched(q_off, n_tok, n_q_heads, g.n_kv_heads);
+    const F32Sched sc = f32_sched(q_off, n_tok, n_q_heads, g.n_kv_heads, D);
     const int hpw = sc.hpw;
     const size_t rows = (size_t)n_tok * n_q_heads;
     if (sc.ksplit > 1 && ws && ws_floats >= (size_t)sc.ksplit * rows * (D + 2)) {
@@ -2316,20 +2329,18 @@ hipError_t launch_prefill_f32(const KvGeom& g, const float* q, const int32_t* pa
     }
     const dim3 grid((unsigned)(g.n_kv_heads * (a.group / hpw)), (unsigned)((n_tok + sc.wrows - 1) / sc.wrows),
                     (unsigned)a.ksplit);
-#define PI_F32(DD)                                                                                \
-    switch (hpw) {                                                                                \
-        case 4: hipLaunchKernelGGL((prefill_f32_kernel<DD, 4>), grid, dim3(512), 0, s, a); break; \
-        case 2: hipLaunchKernelGGL((prefill_f32_kernel<DD, 2>), grid, dim3(512), 0, s, a); break; \
-        default: hipLaunchKernelGGL((prefill_f32_kernel<DD, 1>), grid, dim3(512), 0, s, a);       \
+#define PI_F32(K, DD)                                                                   \
+    switch (hpw) {                                                                      \
+        case 4: hipLaunchKernelGGL((K<DD, 4>), grid, dim3(512), 0, s, a); break;        \
+        case 2: hipLaunchKernelGGL((K<DD, 2>), grid, dim3(512), 0, s, a); break;        \
+        default: hipLaunchKernelGGL((K<DD, 1>), grid, dim3(512), 0, s, a);              \
     }
-    if (D == 256) {
-        switch (hpw) {
-            case 4: hipLaunchKernelGGL(prefill_f32_256_kernel<4>, grid, dim3(512), 0, s, a); break;
-            case 2: hipLaunchKernelGGL(prefill_f32_256_kernel<2>, grid, dim3(512), 0, s, a); break;
-            default: hipLaunchKernelGGL(prefill_f32_256_kernel<1>, grid, dim3(512), 0, s, a);
-        }
-    } else if (D == 128) PI_F32(128)
-    else PI_F32(64)
+    if (D == 256) PI_F32(prefill_f32_16_kernel, 256)
+    else if (sc.rows16) {  // one head a workgroup
+        if (D == 128) hipLaunchKernelGGL((prefill_f32_16_kernel<128, 1>), grid, dim3(512), 0, s, a);
+        else hipLaunchKernelGGL((prefill_f32_16_kernel<64, 1>), grid, dim3(512), 0, s, a);
+    } else if (D == 128) PI_F32(prefill_f32_kernel, 128)
+    else PI_F32(prefill_f32_kernel, 64)
 #undef PI_F32
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || a.ksplit == 1) return e;

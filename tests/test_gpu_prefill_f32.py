@@ -44,6 +44,17 @@ def test_f32_prefill_tile_edges(prev, n, hq, hkv, d):
     _check(c, out, sorted({0, n // 2, n - 1} | {r for r in (31, 32, 63, 64, 127, 128) if r < n}))
 
 
+# 128 keys in all pick the 16-row kernel at every head dim, 129 the 32-row one at 64 and 128
+@pytest.mark.parametrize("hq,hkv", [(8, 2), (3, 3), (5, 2)])
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("prev,n", [(0, 1), (0, 16), (0, 17), (0, 128), (0, 129), (127, 1), (128, 1), (95, 33),
+                                    (96, 33), (50, 64)])
+def test_f32_prefill_short_sequences(prev, n, hq, hkv, d):
+    c = Chunk(np.random.default_rng(prev * 17 + n + hq + d), prev, n, hq, hkv, d)
+    out = c.gpu(device(), pool_dtype=torch.float32)
+    _check(c, out, sorted({0, n // 2, n - 1} | {r for r in (15, 16, 31, 32, 127) if r < n}))
+
+
 @pytest.mark.parametrize("d", [64, 128, 256])
 def test_f32_prefill_max_rises_late(d):
     """Scores that outgrow the running max tile after tile."""
