@@ -1425,18 +1425,19 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_kernel(PrefillArgs a) {
     const int r = lane & 31, hh = lane >> 5;
     const int rg = wave & 3, kh = wave >> 2;
     const int per_kv = a.group / HPW;  // workgroups per KV head and query block
-    const int kvh = (int)blockIdx.x / per_kv;
-    const int head = head_of(kvh, ((int)blockIdx.x % per_kv) * HPW + rg / RG, a.hkv, a.group, a.gqa_mode);
+    const int hset = (int)blockIdx.x % (a.hkv * per_kv), kvh = hset / per_kv;
+    const int head = head_of(kvh, (hset % per_kv) * HPW + rg / RG, a.hkv, a.group, a.gqa_mode);
     // a head that does not exist (modulo map, n_q_heads not a multiple of n_kv_heads: HPW
     // is 1) makes the whole workgroup leave, before any barrier
     if (HPW == 1 && head >= a.hq) return;
-    const int qb = (int)gridDim.y - 1 - (int)blockIdx.y;  // heaviest (latest) query blocks first
+    // x = (query block, head set), the heaviest (latest) blocks first
+    const int qb = (int)(gridDim.x - 1 - blockIdx.x) / (a.hkv * per_kv);
     const int S = a.S, L = a.Sk, q_off = a.q_off;         // L: keys of the sequence after this chunk
     const int p0 = qb * WROWS + 32 * (rg % RG);           // this wave's first query row
     const int qpos = p0 + r;
     // this workgroup's tiles [tb, n_tiles): the block's, or its piece of them under a key split
     const int n_all = (min(L, q_off + qb * WROWS + WROWS) + BN - 1) / BN;  // in 64-key tiles
-    const int ksp = blockIdx.z, pieces = split_pieces(n_all, a.ksplit, a.kthr);
+    const int ksp = blockIdx.y, pieces = split_pieces(n_all, a.ksplit, a.kthr);
     if (ksp >= pieces) return;  // uniform per workgroup
     const int kper = (n_all + pieces - 1) / pieces;
     const int tb = min(n_all, ksp * kper) * (BN / TK);
@@ -1652,16 +1653,17 @@ __global__ __launch_bounds__(512, 2) void prefill_f32_16_kernel(PrefillArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, c = lane & 15;
     const int per_kv = a.group / HPW;           // workgroups per KV head and query block
-    const int kvh = (int)blockIdx.x / per_kv;
-    const int head = head_of(kvh, ((int)blockIdx.x % per_kv) * HPW + wave / RW, a.hkv, a.group, a.gqa_mode);
+    const int hset = (int)blockIdx.x % (a.hkv * per_kv), kvh = hset / per_kv;
+    const int head = head_of(kvh, (hset % per_kv) * HPW + wave / RW, a.hkv, a.group, a.gqa_mode);
     if (HPW == 1 && head >= a.hq) return;  // as in prefill_f32_kernel
-    const int qb = (int)gridDim.y - 1 - (int)blockIdx.y;  // heaviest (latest) query blocks first
+    // x = (query block, head set), the heaviest (latest) blocks first
+    const int qb = (int)(gridDim.x - 1 - blockIdx.x) / (a.hkv * per_kv);
     const int S = a.S, L = a.Sk, q_off = a.q_off;         // L: keys of the sequence after this chunk
     const int p0 = qb * WROWS + 16 * (wave % RW);         // this wave's first query row
     const int qpos = p0 + c;
     // this workgroup's tiles [tb, n_tiles): the block's, or its piece of them under a key split
     const int n_all = (min(L, q_off + qb * WROWS + WROWS) + BN - 1) / BN;  // in 64-key tiles
-    const int ksp = blockIdx.z, pieces = split_pieces(n_all, a.ksplit, a.kthr);
+    const int ksp = blockIdx.y, pieces = split_pieces(n_all, a.ksplit, a.kthr);
     if (ksp >= pieces) return;  // uniform per workgroup
     const int kper = (n_all + pieces - 1) / pieces;
     const int tb = min(n_all, ksp * kper) * (BN / TK);
@@ -2327,8 +2329,10 @@ hipError_t launch_prefill_f32(const KvGeom& g, const float* q, const int32_t* pa
         a.part_o = ws;
         a.part_ml = ws + (size_t)sc.ksplit * rows * D;
     }
-    const dim3 grid((unsigned)(g.n_kv_heads * (a.group / hpw)), (unsigned)((n_tok + sc.wrows - 1) / sc.wrows),
-                    (unsigned)a.ksplit);
+    // the query blocks in x, whose range no prompt exhausts (y and z end at 65 536)
+    const long long wgs = (long long)g.n_kv_heads * (a.group / hpw) * ((n_tok + sc.wrows - 1LL) / sc.wrows);
+    if (wgs * 512 > 0xffffffffLL) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)wgs, (unsigned)a.ksplit);
 #define PI_F32(K, DD)                                                                   \
     switch (hpw) {                                                                      \
         case 4: hipLaunchKernelGGL((K<DD, 4>), grid, dim3(512), 0, s, a); break;        \
