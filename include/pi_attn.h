@@ -20,7 +20,7 @@
  *     the handle's own (non-blocking) stream and synchronise before
  *     returning, like GpuDevice::matvec (src/cuda/mod.rs:244-330);
  *   - one handle per host thread; the library takes no locks.  A handle's
- *     workspaces (decode partials, GDN prefill buffers) may serve calls on
+ *     workspaces (decode and prefill partials, GDN prefill buffers) may serve calls on
  *     different streams: a call on another stream than the previous
  *     workspace user waits (on the device) for that use first;
  *   - all arithmetic is fp32 except where a dtype argument says otherwise;
@@ -188,8 +188,15 @@ int pi_attn_prefill(pi_handle h, const void* d_q, const void* d_k, const void* d
  * (no copy of the history; the handle's workspace holds only the key splits'
  * partials of the chunk's rows).  f32 pool (D = 64, 128 or 256): a kernel
  * reads the pages directly and keeps f32 accuracy (bf16 hi + lo operand splits
- * on the MFMA).  A page id outside [0, n_pages) holds no tokens: its keys are
- * left out of the softmax, as in pi_attn_decode. */
+ * on the MFMA); a call with few rows over many keys splits its keys as the f16
+ * one does, with the partials in the same workspace (which may grow: the call
+ * then waits for the stream and allocates, and calls on two streams of one
+ * handle take turns).  Captured into a graph, or without memory for the
+ * partials, it runs unsplit and touches no workspace: the same sums in another
+ * order, so equal to the split call within f32 rounding but not bit for bit,
+ * and slower by up to the four pieces.  A page id outside [0, n_pages) holds no
+ * tokens: its keys are left out of the softmax, as in pi_attn_decode, and a row
+ * without any other key gets zeros. */
 int pi_attn_prefill_paged(pi_handle h, const void* d_q, pi_kv_pool pool,
                           const int32_t* d_page_table, int32_t max_pages, int32_t start_pos,
                           int32_t n_tok, int32_t n_q_heads, int32_t gqa_mode, float scale,

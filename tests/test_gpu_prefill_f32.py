@@ -1,5 +1,6 @@
-"""The f32 pool's prefill kernels (32-row workgroup tiles with two key halves at head dims 64
-and 128, 16-row ones at 256) at the edges of their tiles, against the oracle.
+"""The f32 pool's prefill kernels (32-row wavefront tiles with two key halves at head dims 64 and
+128, 16-row ones at 256 and for sequences of up to 128 keys) at the edges of their tiles, against
+the oracle.
 
 Tolerance: an operand x is kept as bf16 hi + lo (relative error 2^-17), the lo.lo product is
 dropped (2^-16 of |q_i k_i|), so a score moves by at most e = 2^-15 scale sum_i |q_i k_i|, a
