@@ -2223,7 +2223,7 @@ struct F32Sched {
 constexpr int kF32ShortKeys = 128;
 
 // The f32 prefill's key split.  One workgroup (a block of wrows rows) runs on a CU at a time,
-// about 3 us a 64-key tile, so a launch with fewer blocks than CUs takes its longest block's
+// about 3 us a 64-key tile (D 128, after 10 of launch, first tile, Q and epilogue), so a launch with fewer blocks than CUs takes its longest block's
 // tiles.  Its blocks then run in up to four pieces of at most kthr tiles, the smallest for
 // which all pieces fit the CUs once, if that shortens the longest by the 4 tiles that pay for
 // the merge launch: 64 tokens over 4096, 32/32 heads, D 128 190 -> 64 us, 1024 over 8192 at
