@@ -76,9 +76,6 @@ struct PrefillArgs {
     // every workgroup walks nqb + 1 key tiles and one wave of workgroups fills
     // the chip evenly (else: one block each, heaviest first)
     int paired;
-    // contiguous source: grid y = sequence, z = query block instead of y = query block, z =
-    // (sequence, split); launch_d's choice
-    int seq_fast;
     // key split (a launch with fewer workgroups than CUs): blockIdx.z = batch * ksplit +
     // split.  A query block of n <= kthr key tiles is not split: split 0 takes all its
     // tiles and writes the output, the other splits skip it.  A longer one runs in
@@ -101,6 +98,9 @@ struct PrefillArgs {
     size_t kstride, vstride;
     int n_pages;
     int q_f32;
+    // contiguous source: grid y = sequence, z = query block instead of y = query block, z =
+    // (sequence, split); launch_d's choice
+    int seq_fast;
 };
 
 __device__ __forceinline__ float gate_sigmoid(float g) { return 1.0f / (1.0f + expf(-g)); }
